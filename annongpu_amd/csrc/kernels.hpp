@@ -265,10 +265,14 @@ void launch_gram(const cplx<T>* O, const double* w, int64_t count, int P, cplx<d
 void launch_dense_matvec(const cplx<double>* S, const cplx<double>* x, int P, double shift,
                          cplx<double>* y, hipStream_t stream);
 
-// in-place blocked Cholesky of the lower triangle (fp64 complex, matrix cores); info != 0
-// on failure; work holds cholesky_work_elems() complex values
-size_t cholesky_work_elems();
-void cholesky_lower(cplx<double>* A, int P, int* d_info, cplx<double>* work, hipStream_t stream);
-void cholesky_solve_inplace(const cplx<double>* L, int P, cplx<double>* x, hipStream_t stream);
+// x = (S + shift)^-1 F by a blocked Cholesky of the diagonally scaled matrix (fp64 complex,
+// matrix cores; S, lower triangle read).  A: cholesky_matrix_elems(P) complex values for the
+// factor, work: cholesky_work_elems(P) for the inverses of its diagonal blocks, dinv: P
+// scale factors.  *d_info (zero on entry) holds the 1-based column of the first pivot that
+// is not positive.
+size_t cholesky_matrix_elems(int P);
+size_t cholesky_work_elems(int P);
+void cholesky_solve(const cplx<double>* S, const cplx<double>* F, int P, double shift, cplx<double>* A,
+                    cplx<double>* work, double* dinv, int* d_info, cplx<double>* x, hipStream_t stream);
 
 }  // namespace ann

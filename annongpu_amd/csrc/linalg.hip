@@ -212,240 +212,340 @@ __global__ __launch_bounds__(256) void dense_matvec_kernel(const cplx<double>* S
 }
 
 // -------------------------------------------------------------- Cholesky
-// Right-looking blocked Cholesky of the lower triangle with 64-column panels: the
-// diagonal block is factored (and its triangular inverse formed) in LDS by one
-// workgroup; the panel below it is A L^-H, a matrix-core product with that inverse;
-// the trailing lower tiles take A -= L L^H on matrix cores (K = 64).
-constexpr int kNB = 64;           // panel width (the factor's block size)
-constexpr int kTS = 32;           // block size of the triangular solves
-constexpr int kDL = kNB + 1;      // padded LDS row of the diagonal kernel
+// Solve of (S + shift) x = F by a blocked Cholesky of the diagonally scaled matrix, in a
+// buffer of P + 1 rows: row P holds F^H scaled and takes part in the panel and trailing
+// updates like any other row, so that it ends as (L^-1 F)^H and the forward
+// substitution costs no launch of its own.  64-column blocks: potrf_inv_kernel forms the inverse of
+// the diagonal block's factor in registers; the rows below become A L^-H on matrix
+// cores (ctile_update_kernel<true, ..>); the trailing lower tiles take A -= L L^H
+// (ctile_update_kernel<false, ..>), inside an outer panel of kOuter columns per block (K = 64,
+// the panel's columns only), to the right of it once per outer panel (K = kOuter).
+constexpr int kNB = 64;           // factor block
+// The trailing matrix is read and written once per outer panel: with K = 64 its HBM traffic
+// (16 B in and out per 8 * 64 flop) and not the matrix cores set the time of a large solve.
+// A small one is bound by its chain of launches and skips the second level.
+constexpr int kOuter = 256;
+constexpr int kOuterFrom = 2048;
+constexpr int kCus = 256;         // compute units of an MI355X
 
-// factor the diagonal block A[k:k+nb, k:k+nb] (lower) and write L^-1 to Linv [kNB][kNB]
-__global__ __launch_bounds__(256) void potrf_inv_kernel(cplx<double>* A, int P, int k, int nb, int* info,
+// Scaled copy of the lower triangle: A[i][j] = (S + shift)[i][j] dinv_i dinv_j, j <= i,
+// dinv_i = (S_ii + shift)^-1/2 (1 where that is not positive), and row P = (dinv F)^H.
+// The scaled matrix has the same solution and a far smaller condition number when the
+// parameters' scales differ.
+__global__ __launch_bounds__(256) void chol_scale_kernel(const cplx<double>* S, const cplx<double>* F, int P,
+                                                         double shift, double* dinv, cplx<double>* A) {
+    const int cols = (P + 255) / 256;   // column blocks of a row
+    const int i = int(blockIdx.x / cols), j0 = int(blockIdx.x % cols) * 256;
+    const int j = j0 + threadIdx.x;
+    if (j0 > i || j >= P) return;
+    auto scale = [&](int r) {
+        const double d = S[int64_t(r) * P + r].re + shift;
+        return d > 0.0 ? 1.0 / sqrt(d) : 1.0;
+    };
+    const double fj = scale(j);
+    if (i == P) {
+        dinv[j] = fj;
+        A[int64_t(P) * P + j] = {F[j].re * fj, -F[j].im * fj};
+        return;
+    }
+    if (j > i) return;
+    const cplx<double> a = S[int64_t(i) * P + j];
+    const double f = fj * scale(i);
+    A[int64_t(i) * P + j] = {(i == j ? a.re + shift : a.re) * f, a.im * f};
+}
+
+// The inverse Linv [kNB][kNB] of the factor of the diagonal block A[k:k+nb, k:k+nb] (lower);
+// the factor itself is read by nothing and not stored.  One workgroup, bound by its chain of
+// dependent steps, so the block stays in registers as matrix-core accumulators (both
+// triangles; wave w holds rows 16 w .. 16 w + 15) and four pivots are taken per step: the four
+// rows of a step are one accumulator item of their wave, they go through LDS (one barrier),
+// every wave that still has rows factors the 4 x 4 block and substitutes the rows by itself,
+// one column a lane (right of the block conj(L), left of it the rows of the inverse so far,
+// in it the inverse of the 4 x 4 factor), and the rows below take the rank-4 update as one
+// K = 4 matrix product.  The block's columns start from zero there and become columns of the
+// inverse, in place, as in a Gauss-Jordan inversion.
+// A 64 x 64 block: 128 us with the block in LDS, an element-wise update and three barriers a
+// pivot; 48 us in registers with one pivot a barrier; 34 us here.
+__global__ __launch_bounds__(256) void potrf_inv_kernel(const cplx<double>* A, int P, int k, int nb, int* info,
                                                         cplx<double>* Linv) {
-    extern __shared__ double dl[];
-    double* Lr = dl;                  // [kNB][kDL]
-    double* Li = dl + kNB * kDL;
-    double* Xr = dl + 2 * kNB * kDL;
-    double* Xi = dl + 3 * kNB * kDL;
-    for (int e = threadIdx.x; e < nb * nb; e += 256) {
-        const int i = e / nb, j = e % nb;
-        const cplx<double> a = A[int64_t(k + i) * P + k + j];
-        Lr[i * kDL + j] = a.re;
-        Li[i * kDL + j] = a.im;
-    }
-    __syncthreads();
-    for (int j = 0; j < nb; j++) {
-        if (threadIdx.x == 0) {
-            const double d = Lr[j * kDL + j];
+    __shared__ double2 row[2][4][kNB];   // the step's rows
+    __shared__ double2 ysh[4][4][kNB];   // each wave's substituted rows
+    const int lane = threadIdx.x & 63, w = uniform_int(threadIdx.x >> 6);
+    const int lc = lane & 15, lk = lane >> 4;
+    double4_t re[4], im[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = 16 * w + lk + 4 * i, c = 16 * u + lc, hi = r > c ? r : c, lo = r > c ? c : r;
+            cplx<double> x = {0.0, 0.0};
+            if (hi < nb) x = A[int64_t(k + hi) * P + k + lo];
+            re[u][i] = x.re;
+            im[u][i] = c > r ? -x.im : x.im;
+        }
+#pragma unroll 1   // (sixteen copies of the step would run from cold instruction lines)
+    for (int t = 0; 4 * t < nb; t++) {
+        const int j0 = 4 * t, owner = t >> 2, rr = t & 3, b = t & 1;
+        if (w == owner) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (i == rr) {
+#pragma unroll
+                    for (int u = 0; u < 4; u++) row[b][lk][16 * u + lc] = double2{re[u][i], im[u][i]};
+                }
+        }
+        __syncthreads();   // double-buffered: the next write of buffer b follows the next barrier
+        if (w < owner) continue;   // (wave-uniform) all rows finished
+        double2 y[4], u_[4][4];    // u_[q][s], s >= q: entry (j0 + q, j0 + s)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            y[q] = row[b][q][lane];
+#pragma unroll
+            for (int s = q; s < 4; s++) u_[q][s] = row[b][q][j0 + s];
+        }
+        const int in = lane - j0;
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (in >= 0 && in < 4) y[q] = double2{in == q && j0 + q < nb ? 1.0 : 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            double d = u_[q][q].x;
             if (!(d > 0.0)) {
-                atomicCAS(info, 0, k + j + 1);
-                Lr[j * kDL + j] = 1.0;
-            } else {
-                Lr[j * kDL + j] = sqrt(d);
+                if (j0 + q < nb && threadIdx.x == 64 * owner) atomicCAS(info, 0, k + j0 + q + 1);
+                d = 1.0;
             }
-            Li[j * kDL + j] = 0.0;
-        }
-        __syncthreads();
-        const double inv = 1.0 / Lr[j * kDL + j];
-        for (int i = j + 1 + threadIdx.x; i < nb; i += 256) {
-            Lr[i * kDL + j] *= inv;
-            Li[i * kDL + j] *= inv;
-        }
-        __syncthreads();
-        // trailing update A[i][l] -= L[i][j] conj(L[l][j]), j < l <= i
-        const int rem = nb - j - 1;
-        for (int e = threadIdx.x; e < rem * rem; e += 256) {
-            const int i = j + 1 + e / rem, l = j + 1 + e % rem;
-            if (l <= i) {
-                const double ar = Lr[i * kDL + j], ai = Li[i * kDL + j], br = Lr[l * kDL + j], bi = -Li[l * kDL + j];
-                Lr[i * kDL + l] -= ar * br - ai * bi;
-                Li[i * kDL + l] -= ar * bi + ai * br;
+            const double inv = rsqrt(d);
+            y[q].x *= inv;
+            y[q].y *= inv;
+#pragma unroll
+            for (int s = q + 1; s < 4; s++) {
+                u_[q][s].x *= inv;   // conj(L_sq)
+                u_[q][s].y *= inv;
             }
-        }
-        __syncthreads();
-    }
-    // X = L^-1 by forward substitution, four threads per column (partial sums over m
-    // interleaved by 4, combined by shuffles within the quad)
-    const int col = threadIdx.x >> 2, part = threadIdx.x & 3;
-    for (int i = 0; i < nb; i++) {
-        double sr = 0.0, si = 0.0;
-        if (col < nb && i >= col)
-            for (int m = col + part; m < i; m += 4) {
-                const double lr = Lr[i * kDL + m], li = Li[i * kDL + m], xr = Xr[m * kDL + col], xi = Xi[m * kDL + col];
-                sr += lr * xr - li * xi;
-                si += lr * xi + li * xr;
-            }
-        sr += __shfl_xor(sr, 1);
-        si += __shfl_xor(si, 1);
-        sr += __shfl_xor(sr, 2);
-        si += __shfl_xor(si, 2);
-        if (col < nb && part == 0) {
-            const double d = Lr[i * kDL + i];   // real, positive
-            if (i < col) {
-                Xr[i * kDL + col] = 0.0;
-                Xi[i * kDL + col] = 0.0;
-            } else {
-                Xr[i * kDL + col] = ((i == col ? 1.0 : 0.0) - sr) / d;
-                Xi[i * kDL + col] = -si / d;
+            // rows s > q lose L_sq = conj(u_qs) times row q
+#pragma unroll
+            for (int s = q + 1; s < 4; s++) {
+                const double lr = u_[q][s].x, li = -u_[q][s].y;
+#pragma unroll
+                for (int v = s; v < 4; v++) {
+                    u_[s][v].x = fma(-lr, u_[q][v].x, fma(li, u_[q][v].y, u_[s][v].x));
+                    u_[s][v].y = fma(-lr, u_[q][v].y, fma(-li, u_[q][v].x, u_[s][v].y));
+                }
+                y[s].x = fma(-lr, y[q].x, fma(li, y[q].y, y[s].x));
+                y[s].y = fma(-lr, y[q].y, fma(-li, y[q].x, y[s].y));
             }
         }
-        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4; q++) ysh[w][q][lane] = y[q];
+        // operands of A_rc -= sum_q L_r,j0+q y_qc (L_r,j0+q = conj(y_qr), rows below the block)
+        const double2 yr = ysh[w][lk][16 * w + lc];
+        const bool below = 16 * w + lc > j0 + 3;
+        const double ar = below ? -yr.x : 0.0, ai = below ? yr.y : 0.0;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const double2 yc = ysh[w][lk][16 * u + lc];
+            if (u == owner && (lc >> 2) == rr) {
+                re[u] = {0.0, 0.0, 0.0, 0.0};
+                im[u] = {0.0, 0.0, 0.0, 0.0};
+            }
+            re[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, yc.x, re[u], 0, 0, 0);
+            im[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, yc.y, im[u], 0, 0, 0);
+            re[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, yc.y, re[u], 0, 0, 0);
+            im[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, yc.x, im[u], 0, 0, 0);
+            if (w == owner) {   // the block's own rows
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (i == rr) {
+                        re[u][i] = yc.x;
+                        im[u][i] = yc.y;
+                    }
+            }
+        }
     }
-    for (int e = threadIdx.x; e < nb * nb; e += 256) {
-        const int i = e / nb, j = e % nb;
-        if (j <= i) A[int64_t(k + i) * P + k + j] = {Lr[i * kDL + j], Li[i * kDL + j]};
-    }
-    for (int e = threadIdx.x; e < kNB * kNB; e += 256) {
-        const int i = e / kNB, j = e % kNB;
-        Linv[e] = i < nb && j < nb ? cplx<double>{Xr[i * kDL + j], Xi[i * kDL + j]} : cplx<double>{0.0, 0.0};
-    }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = 16 * w + lk + 4 * i, c = 16 * u + lc;
+            Linv[r * kNB + c] = r < nb && c <= r ? cplx<double>{re[u][i], im[u][i]} : cplx<double>{0.0, 0.0};
+        }
 }
 
-// panel rows r0 + 64 blockIdx.x ..: A[i, k:k+nb] <- A[i, k:k+nb] L^-H (in place: every
-// stage is read before the tile is written)
-__global__ __launch_bounds__(256) void panel_mfma_kernel(cplx<double>* A, int P, int k, int nb, int r0,
-                                                         const cplx<double>* Linv) {
-    extern __shared__ double lds[];   // [kNB / kCS][kCStage]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wr = wave >> 1, wc = wave & 1;
-    const int rb = r0 + blockIdx.x * kCT;
-    for (int e = threadIdx.x; e < kNB * kCT; e += 256) {
-        const int i = e / kNB, m = e % kNB;   // A operand [m][i] = A[rb + i][k + m] (rows read contiguously)
-        double* st = lds + (m / kCS) * kCStage;
-        const int o = (m % kCS) * kCT + i;
-        cplx<double> a = {0.0, 0.0};
-        if (m < nb && rb + i < P) a = A[int64_t(rb + i) * P + k + m];
-        st[o] = a.re;
-        st[kCS * kCT + o] = a.im;
-        // B operand [m][j] = conj(Linv[j][m])
-        const cplx<double> b = Linv[i * kNB + m];
-        st[2 * kCS * kCT + o] = b.re;
-        st[3 * kCS * kCT + o] = -b.im;
+// Complex tiles of A (rows below, ld = P, `rows` rows), K values of k in stages of KS:
+//   SOLVE:  A[i][k0+j] <- sum_m A[i][k0+m] conj(Linv[j][m]) for the rows from s0 (in place: a
+//           tile spans the block's columns and its rows are read whole before they are written)
+//   else:   A[i][j] -= sum_m A[i][k0+m] conj(A[j][k0+m]), j <= i, for the row tiles from s0 and
+//           the column tiles from s0 below cend (every pair of the triangle when ctiles == 0)
+// Four waves as WR x (4 / WR), T x T matrix-core tiles of 16 x 16 each.  Both operands are rows
+// read along m; they are staged as complex [row][KS] with a row of KS + 1 (a 16-row fragment
+// then takes 16 different 16-byte bank groups; the operands transposed into [m][row] put a
+// wave's 64 writes into one bank).  KS = 64 holds all of a K = 64 product, whose loads are then
+// one memory round trip; KS = 16 is double-buffered, the next stage's global loads in flight
+// during the matrix instructions.  A 64 x 64 tile of K = 64 keeps one CU's matrix cores busy
+// for 7 us, so where the tiles do not fill the chip smaller ones shorten the chain of launches.
+template <int KS, int WR, int T>
+struct UpdateTile {
+    static constexpr int kRows = 16 * T * WR, kCols = 16 * T * (4 / WR);
+    static constexpr int kRow = KS + 1;   // padded complex row
+    static constexpr int kBuf = (kRows + kCols) * kRow;
+    static constexpr size_t kLds = sizeof(double2) * (KS == kNB ? 1 : 2) * kBuf;
+};
+template <bool SOLVE, int KS, int WR, int T>
+__global__ __launch_bounds__(256) void ctile_update_kernel(cplx<double>* A, int P, int rows, int k0, int K, int s0,
+                                                           int ctiles, int cend, int64_t tiles,
+                                                           const cplx<double>* Linv) {
+    using U = UpdateTile<KS, WR, T>;
+    static_assert(SOLVE ? U::kCols == kNB : U::kRows == U::kCols, "tile shape");
+    constexpr int WC = 4 / WR;
+    extern __shared__ double2 ust[];   // [buffers][kRows of A, kCols of the second operand][kRow]
+    int bi, bj = 0;
+    if constexpr (SOLVE) {
+        bi = blockIdx.x;
+    } else if (ctiles > 0) {
+        bj = int(blockIdx.x) % ctiles;
+        bi = int(blockIdx.x) / ctiles;
+        if (bi < bj) return;
+    } else {
+        const int64_t t = xcd_tile(blockIdx.x, tiles);
+        if (t >= tiles) return;
+        upper_pair(t, bj, bi);   // bj <= bi
     }
-    __syncthreads();
-    CTileAcc acc;
-    ctile_zero(acc);
-    for (int g = 0; g < kNB / kCS; g++) ctile_stage(lds + g * kCStage, lane, wr, wc, acc);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wr = wave / WC, wc = wave % WC;
+    const int r0 = s0 + bi * U::kRows, c0 = SOLVE ? 0 : s0 + bj * U::kCols;
+    constexpr int kStep = 256 / KS;                              // rows per load round
+    constexpr int kA = U::kRows / kStep, kB = U::kCols / kStep;  // loads per thread
+    const int lm = threadIdx.x & (KS - 1), lr = threadIdx.x / KS;
+    double2 fa[kA], fb[kB];
+    auto load_row = [&](int r, int m) {
+        return m < K && r < rows ? *reinterpret_cast<const double2*>(A + int64_t(r) * P + k0 + m) : double2{0.0, 0.0};
+    };
+    auto fetch = [&](int g) {
+        const int m = g * KS + lm;
 #pragma unroll
-    for (int t = 0; t < 2; t++)
+        for (int e = 0; e < kA; e++) fa[e] = load_row(r0 + lr + kStep * e, m);
 #pragma unroll
-        for (int u = 0; u < 2; u++)
+        for (int e = 0; e < kB; e++) {
+            const int r = c0 + lr + kStep * e;
+            if constexpr (SOLVE)
+                fb[e] = *reinterpret_cast<const double2*>(Linv + r * kNB + m);
+            else
+                fb[e] = load_row(r, m);
+        }
+    };
+    auto stash = [&](int buf) {
+        double2* st = ust + buf * U::kBuf;
+#pragma unroll
+        for (int e = 0; e < kA; e++) st[(lr + kStep * e) * U::kRow + lm] = fa[e];
+#pragma unroll
+        for (int e = 0; e < kB; e++) st[(U::kRows + lr + kStep * e) * U::kRow + lm] = fb[e];
+    };
+    // f64 16x16x4 result layout: item r of lane l is row l/16 + 4 r, column l%16
+    auto row_of = [&](int t, int r) { return r0 + (wr * T + t) * 16 + (lane >> 4) + 4 * r; };
+    auto col_of = [&](int u) { return c0 + (wc * T + u) * 16 + (lane & 15); };
+    const int stages = (K + KS - 1) / KS;
+    fetch(0);
+    double4_t re[T][T], im[T][T];
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int u = 0; u < T; u++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int gr = rb + ctile_row(lane, wr, t, r), j = ctile_col(lane, wc, u);
-                if (gr < P && j < nb) A[int64_t(gr) * P + k + j] = {acc.re[t][u][r], acc.im[t][u][r]};
+                cplx<double> x = {0.0, 0.0};
+                const int gi = row_of(t, r), gj = col_of(u);
+                if (!SOLVE && gi < rows && gj <= gi && gj < cend) x = A[int64_t(gi) * P + gj];
+                re[t][u][r] = -x.re;
+                im[t][u][r] = -x.im;
             }
-}
-
-// trailing update of the lower 64 x 64 tiles (bi >= bj) from s0:
-// A[i][j] -= sum_m A[i][k+m] conj(A[j][k+m])
-__global__ __launch_bounds__(256) void herk_mfma_kernel(cplx<double>* A, int P, int k, int nb, int s0,
-                                                        int64_t pairs) {
-    extern __shared__ double lds[];   // [kNB / kCS][kCStage]
-    const int64_t t = xcd_tile(blockIdx.x, pairs);
-    if (t >= pairs) return;
-    int bj, bi;
-    upper_pair(t, bj, bi);   // bj <= bi
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wr = wave >> 1, wc = wave & 1;
-    const int r0 = s0 + bi * kCT, c0 = s0 + bj * kCT;
-    for (int e = threadIdx.x; e < kNB * kCT; e += 256) {
-        const int i = e / kNB, m = e % kNB;   // rows of the panel read contiguously
-        double* st = lds + (m / kCS) * kCStage;
-        const int o = (m % kCS) * kCT + i;
-        cplx<double> x = {0.0, 0.0}, y = {0.0, 0.0};
-        if (m < nb && r0 + i < P) x = A[int64_t(r0 + i) * P + k + m];
-        if (m < nb && c0 + i < P) y = A[int64_t(c0 + i) * P + k + m];
-        st[o] = x.re;
-        st[kCS * kCT + o] = x.im;
-        st[2 * kCS * kCT + o] = y.re;       // B [m][j] = conj(A[c0 + j][k + m])
-        st[3 * kCS * kCT + o] = -y.im;
-    }
+    stash(0);
     __syncthreads();
-    CTileAcc acc;
-    ctile_zero(acc);
-    for (int g = 0; g < kNB / kCS; g++) ctile_stage(lds + g * kCStage, lane, wr, wc, acc);
+    for (int g = 0; g < stages; g++) {
+        if (g + 1 < stages) fetch(g + 1);
+        const double2* As = ust + (KS == kNB ? 0 : g & 1) * U::kBuf;
+        const double2* Bs = As + U::kRows * U::kRow;
 #pragma unroll
-    for (int tt = 0; tt < 2; tt++)
+        for (int q = 0; q < KS / 4; q++) {
+            const int kk = 4 * q + (lane >> 4);
+            double2 a[T], b[T];
 #pragma unroll
-        for (int u = 0; u < 2; u++)
+            for (int t = 0; t < T; t++) {
+                a[t] = As[((wr * T + t) * 16 + (lane & 15)) * U::kRow + kk];
+                b[t] = Bs[((wc * T + t) * 16 + (lane & 15)) * U::kRow + kk];
+            }
+            // A times the conjugate of the second operand's rows
+#pragma unroll
+            for (int t = 0; t < T; t++)
+#pragma unroll
+                for (int u = 0; u < T; u++) {
+                    re[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t].x, b[u].x, re[t][u], 0, 0, 0);
+                    im[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t].y, b[u].x, im[t][u], 0, 0, 0);
+                    re[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t].y, b[u].y, re[t][u], 0, 0, 0);
+                    im[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[t].x, b[u].y, im[t][u], 0, 0, 0);
+                }
+        }
+        if (g + 1 < stages) stash((g + 1) & 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int u = 0; u < T; u++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int gi = r0 + ctile_row(lane, wr, tt, r), gj = c0 + ctile_col(lane, wc, u);
-                if (gi < P && gj <= gi) {
-                    cplx<double>& dst = A[int64_t(gi) * P + gj];
-                    dst.re -= acc.re[tt][u][r];
-                    dst.im -= acc.im[tt][u][r];
+                const int gi = row_of(t, r), gj = col_of(u);
+                if constexpr (SOLVE) {
+                    if (gi < rows && gj < K) A[int64_t(gi) * P + k0 + gj] = {re[t][u][r], im[t][u][r]};
+                } else {
+                    if (gi < rows && gj <= gi && gj < cend)
+                        A[int64_t(gi) * P + gj] = {-re[t][u][r], -im[t][u][r]};
                 }
             }
 }
 
-// forward: solve L_kk y_k = b_k in place (one block), then b_i -= L_ik y_k for i > block
-__global__ __launch_bounds__(256) void trsv_lower_block_kernel(const cplx<double>* L, int P, int k, int nb,
-                                                               cplx<double>* x) {
-    __shared__ double yr[kTS], yi[kTS];
-    if (threadIdx.x == 0) {
-        for (int j = 0; j < nb; j++) {
-            double r = x[k + j].re, im = x[k + j].im;
-            for (int m = 0; m < j; m++) {
-                const cplx<double> l = L[int64_t(k + j) * P + k + m];
-                r -= l.re * yr[m] - l.im * yi[m];
-                im -= l.re * yi[m] + l.im * yr[m];
-            }
-            const double d = L[int64_t(k + j) * P + k + j].re;
-            yr[j] = r / d;
-            yi[j] = im / d;
-            x[k + j] = {yr[j], yi[j]};
-        }
+// One block of the backward substitution L^H x = y, in conjugated form on row P of A (y^H on
+// entry): x'_j = sum_m Linv[m][j] y'_m for the block's columns, then y'_i -= sum_m L[k+m][i] x'_m
+// for the 64 columns i < k of this workgroup, and x = conj(x') dinv.  Every workgroup forms the
+// block's x' itself (64 KB of Linv from L2), so a block is one launch; its rows of L are in
+// flight meanwhile.  (A single-thread triangular solve of 32 columns took 28-51 us a block.)
+__global__ __launch_bounds__(256) void chol_back_kernel(cplx<double>* A, int P, int k, int nb,
+                                                        const cplx<double>* Linv, const double* dinv,
+                                                        cplx<double>* x) {
+    __shared__ cplx<double> sy[kNB], sx[kNB], part[4][kNB];
+    const int c = threadIdx.x & 63, q = threadIdx.x >> 6;
+    cplx<double>* row = A + int64_t(P) * P;
+    const int i = blockIdx.x * 64 + c;
+    cplx<double> l[16];
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        const int m = q * 16 + e;
+        l[e] = i < k && m < nb ? A[int64_t(k + m) * P + i] : cplx<double>{0.0, 0.0};
     }
-}
-__global__ __launch_bounds__(256) void gemv_lower_update_kernel(const cplx<double>* L, int P, int k, int nb,
-                                                                cplx<double>* x) {
-    const int i = k + nb + blockIdx.x * 256 + threadIdx.x;
-    if (i >= P) return;
-    double r = 0, im = 0;
-    for (int m = 0; m < nb; m++) {
-        const cplx<double> l = L[int64_t(i) * P + k + m];
-        const cplx<double> y = x[k + m];
-        r += l.re * y.re - l.im * y.im;
-        im += l.re * y.im + l.im * y.re;
+    if (q == 0) sy[c] = c < nb ? row[k + c] : cplx<double>{0.0, 0.0};
+    __syncthreads();
+    cplx<double> s = {0.0, 0.0};
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        const int m = q * 16 + e;
+        s = cadd(s, cmul(Linv[m * kNB + c], sy[m]));
     }
-    x[i].re -= r;
-    x[i].im -= im;
-}
-// backward: solve L_kk^H x_k = y_k, then y_i -= sum_m conj(L[k+m][i]) x_{k+m} for i < k
-__global__ __launch_bounds__(256) void trsv_upper_block_kernel(const cplx<double>* L, int P, int k, int nb,
-                                                               cplx<double>* x) {
-    __shared__ double zr[kTS], zi[kTS];
-    if (threadIdx.x == 0) {
-        for (int j = nb - 1; j >= 0; j--) {
-            double r = x[k + j].re, im = x[k + j].im;
-            for (int m = j + 1; m < nb; m++) {
-                const cplx<double> l = L[int64_t(k + m) * P + k + j];   // conj(L[m][j]) * z_m
-                r -= l.re * zr[m] + l.im * zi[m];
-                im -= l.re * zi[m] - l.im * zr[m];
-            }
-            const double d = L[int64_t(k + j) * P + k + j].re;
-            zr[j] = r / d;
-            zi[j] = im / d;
-            x[k + j] = {zr[j], zi[j]};
-        }
+    part[q][c] = s;
+    __syncthreads();
+    if (q == 0) {
+        s = cadd(cadd(part[0][c], part[1][c]), cadd(part[2][c], part[3][c]));
+        sx[c] = s;
+        if (blockIdx.x == 0 && c < nb) x[k + c] = {s.re * dinv[k + c], -s.im * dinv[k + c]};
     }
-}
-__global__ __launch_bounds__(256) void gemv_upper_update_kernel(const cplx<double>* L, int P, int k, int nb,
-                                                                cplx<double>* x) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= k) return;
-    double r = 0, im = 0;
-    for (int m = 0; m < nb; m++) {
-        const cplx<double> l = L[int64_t(k + m) * P + i];
-        const cplx<double> z = x[k + m];
-        r += l.re * z.re + l.im * z.im;
-        im += l.re * z.im - l.im * z.re;
+    __syncthreads();
+    s = {0.0, 0.0};
+#pragma unroll
+    for (int e = 0; e < 16; e++) s = cadd(s, cmul(l[e], sx[q * 16 + e]));
+    part[q][c] = s;   // (the first use of part is over: sx was formed from it)
+    __syncthreads();
+    if (q == 0 && i < k) {
+        s = cadd(cadd(part[0][c], part[1][c]), cadd(part[2][c], part[3][c]));
+        row[i] = csub(row[i], s);
     }
-    x[i].re -= r;
-    x[i].im -= im;
 }
 
 }  // namespace
@@ -476,52 +576,58 @@ void launch_dense_matvec(const cplx<double>* S, const cplx<double>* x, int P, do
     ANN_LAUNCH_CHECK();
 }
 
-size_t cholesky_work_elems() { return size_t(kNB) * kNB; }
+size_t cholesky_matrix_elems(int P) { return size_t(P + 1) * P; }
+size_t cholesky_work_elems(int P) { return size_t((P + kNB - 1) / kNB) * kNB * kNB; }
 
-void cholesky_lower(cplx<double>* A, int P, int* d_info, cplx<double>* work, hipStream_t stream) {
-    const size_t diag_lds = sizeof(double) * 4 * kNB * kDL;
-    const size_t tile_lds = sizeof(double) * (kNB / kCS) * kCStage;   // 128 KiB
-    ANN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(potrf_inv_kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(diag_lds)));
-    ANN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(panel_mfma_kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(tile_lds)));
-    ANN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(herk_mfma_kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(tile_lds)));
-    for (int k = 0; k < P; k += kNB) {
+void cholesky_solve(const cplx<double>* S, const cplx<double>* F, int P, double shift, cplx<double>* A,
+                    cplx<double>* work, double* dinv, int* d_info, cplx<double>* x, hipStream_t stream) {
+    if (P <= 0) return;
+    chol_scale_kernel<<<unsigned((P + 255) / 256) * unsigned(P + 1), 256, 0, stream>>>(S, F, P, shift, dinv, A);
+    ANN_LAUNCH_CHECK();
+    const int rows = P + 1;
+    const int outer = P >= kOuterFrom ? kOuter : kNB;
+    auto launch = [&](auto kernel, size_t lds, int64_t grid, auto... args) {
+        ANN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+        kernel<<<unsigned(grid), 256, lds, stream>>>(A, P, rows, args...);
+        ANN_LAUNCH_CHECK();
+    };
+    auto tiles = [](int n, int t) { return int64_t((n + t - 1) / t); };
+    // the columns [s0, cend) of the rows from s0 take the product of the columns [k, k + K)
+    auto update = [&](int k, int K, int s0, int cend) {
+        const bool tri = cend == P;   // the whole trailing triangle
+        auto run = [&](auto kernel, size_t lds, int tile) {
+            const int64_t nt = tiles(rows - s0, tile), ct = tiles(cend - s0, tile), pairs = nt * (nt + 1) / 2;
+            launch(kernel, lds, tri ? (pairs + 7) / 8 * 8 : nt * ct, k, K, s0, tri ? 0 : int(ct), cend, pairs,
+                   static_cast<const cplx<double>*>(nullptr));
+        };
+        const int64_t nt64 = tiles(rows - s0, 64), n64 = tri ? nt64 * (nt64 + 1) / 2 : nt64 * tiles(cend - s0, 64);
+        if (K > kNB)
+            run(ctile_update_kernel<false, 16, 2, 2>, UpdateTile<16, 2, 2>::kLds, 64);
+        else if (n64 < kCus)
+            run(ctile_update_kernel<false, kNB, 2, 1>, UpdateTile<kNB, 2, 1>::kLds, 32);
+        else
+            run(ctile_update_kernel<false, kNB, 2, 2>, UpdateTile<kNB, 2, 2>::kLds, 64);
+    };
+    for (int p = 0; p < P; p += outer) {
+        const int pend = P - p < outer ? P : p + outer;
+        for (int k = p; k < pend; k += kNB) {
+            const int nb = pend - k < kNB ? pend - k : kNB;
+            const int s0 = k + nb;
+            cplx<double>* Linv = work + int64_t(k / kNB) * kNB * kNB;
+            potrf_inv_kernel<<<1, 256, 0, stream>>>(A, P, k, nb, d_info, Linv);
+            ANN_LAUNCH_CHECK();
+            launch(ctile_update_kernel<true, kNB, 1, 1>, UpdateTile<kNB, 1, 1>::kLds, tiles(rows - s0, 16), k, nb, s0,
+                   0, 0, int64_t(0), static_cast<const cplx<double>*>(Linv));
+            if (s0 < pend) update(k, nb, s0, pend);
+        }
+        if (pend < P) update(p, pend - p, pend, P);
+    }
+    for (int k = (P - 1) / kNB * kNB; k >= 0; k -= kNB) {
         const int nb = P - k < kNB ? P - k : kNB;
-        potrf_inv_kernel<<<1, 256, diag_lds, stream>>>(A, P, k, nb, d_info, work);
+        chol_back_kernel<<<unsigned(k > 0 ? tiles(k, 64) : 1), 256, 0, stream>>>(
+            A, P, k, nb, work + int64_t(k / kNB) * kNB * kNB, dinv, x);
         ANN_LAUNCH_CHECK();
-        const int s0 = k + nb, rest = P - s0;
-        if (rest <= 0) break;
-        panel_mfma_kernel<<<unsigned((rest + kCT - 1) / kCT), 256, tile_lds, stream>>>(A, P, k, nb, s0, work);
-        ANN_LAUNCH_CHECK();
-        const int64_t nt = (rest + kCT - 1) / kCT;
-        const int64_t pairs = nt * (nt + 1) / 2;
-        herk_mfma_kernel<<<unsigned((pairs + 7) / 8 * 8), 256, tile_lds, stream>>>(A, P, k, nb, s0, pairs);
-        ANN_LAUNCH_CHECK();
-    }
-}
-
-void cholesky_solve_inplace(const cplx<double>* L, int P, cplx<double>* x, hipStream_t stream) {
-    for (int k = 0; k < P; k += kTS) {
-        const int nb = P - k < kTS ? P - k : kTS;
-        trsv_lower_block_kernel<<<1, 64, 0, stream>>>(L, P, k, nb, x);
-        ANN_LAUNCH_CHECK();
-        const int rest = P - k - nb;
-        if (rest > 0) {
-            gemv_lower_update_kernel<<<unsigned((rest + 255) / 256), 256, 0, stream>>>(L, P, k, nb, x);
-            ANN_LAUNCH_CHECK();
-        }
-    }
-    const int last = ((P - 1) / kTS) * kTS;
-    for (int k = last; k >= 0; k -= kTS) {
-        const int nb = P - k < kTS ? P - k : kTS;
-        trsv_upper_block_kernel<<<1, 64, 0, stream>>>(L, P, k, nb, x);
-        ANN_LAUNCH_CHECK();
-        if (k > 0) {
-            gemv_upper_update_kernel<<<unsigned((k + 255) / 256), 256, 0, stream>>>(L, P, k, nb, x);
-            ANN_LAUNCH_CHECK();
-        }
     }
 }
 

@@ -1866,26 +1866,15 @@ int tdvp_solve(Tdvp& t, double shift, int method, double rtol, int max_iter, cd*
         x.ensure(P);
         if (!t.has_S) throw std::logic_error("Cholesky solve needs TDVP.eval with the S matrix");
         // the factor and its workspace persist in the TDVP object (4.5 GB at P = 16,704)
-        DevBuf<cplx<double>>& A = t.chol;
-        A.ensure(size_t(P) * P);
-        t.chol_work.ensure(cholesky_work_elems());
+        t.chol.ensure(cholesky_matrix_elems(P));
+        t.chol_work.ensure(cholesky_work_elems(P));
+        t.chol_dinv.ensure(P);
         DevBuf<int> info;
         info.ensure(1);
         ANN_HIP_CHECK(hipMemsetAsync(info.p, 0, sizeof(int), S()));
-        ANN_HIP_CHECK(hipMemcpyAsync(A.p, t.S.p, sizeof(cplx<double>) * P * P, hipMemcpyDeviceToDevice, S()));
         {
             ScopedTimer timer("cholesky");
-            launch_add_diag(A.p, P, shift, S());
-            // factor the diagonally scaled matrix (same solution, far smaller condition
-            // number when the O_k of different parameters differ in scale)
-            DevBuf<double>& dinv = t.chol_dinv;
-            dinv.ensure(P);
-            launch_equilibrate(A.p, P, dinv.p, S());
-            cholesky_lower(A.p, P, info.p, t.chol_work.p, S());
-            ANN_HIP_CHECK(hipMemcpyAsync(x.p, t.Fd.p, sizeof(cplx<double>) * P, hipMemcpyDeviceToDevice, S()));
-            launch_scale_vec(x.p, P, dinv.p, S());
-            cholesky_solve_inplace(A.p, P, x.p, S());
-            launch_scale_vec(x.p, P, dinv.p, S());
+            cholesky_solve(t.S.p, t.Fd.p, P, shift, t.chol.p, t.chol_work.p, t.chol_dinv.p, info.p, x.p, S());
         }
         int hinfo = 0;
         ANN_HIP_CHECK(hipMemcpyAsync(&hinfo, info.p, sizeof(int), hipMemcpyDeviceToHost, S()));
