@@ -256,10 +256,20 @@ void launch_kl_terms(const cplx<double>* lp, const cplx<double>* lpp, const doub
                      cplx<double> last_mean_deviation, double threshold, cplx<double>* c_w, cplx<double>* c_d,
                      cplx<double>* c_d2, double* sums6, hipStream_t stream);
 
-// dense Hermitian Gram S = O^H diag(w) O  (O row-major [count][P], complex T)
+// dense Hermitian Gram S = O^H diag(w) O  (O row-major [count][P], complex T); work:
+// gram_work_elems complex values (none are needed when it is 0)
+size_t gram_work_elems(int P, int64_t count);
 template <typename T>
-void launch_gram(const cplx<T>* O, const double* w, int64_t count, int P, cplx<double>* S,
+void launch_gram(const cplx<T>* O, const double* w, int64_t count, int P, cplx<double>* work, cplx<double>* S,
                  hipStream_t stream);
+
+// the same for a one-layer net from g and the transposed spin bits (row N all ones), less
+// conj(<O>) <O> (gram_dense.hip); work: dense_gram_work_elems doubles, mean: <O>, P values
+size_t dense_gram_work_elems(int N, int M, int64_t count);
+template <typename T>
+void launch_dense_gram(int layout, int N, int M, int Mpad, const uint32_t* conn, const uint64_t* bits, int vpad,
+                       const cplx<T>* g, const double* w, int64_t count, int P, double* work, cplx<double>* mean,
+                       cplx<double>* S, hipStream_t stream);
 
 // y = S x for dense S in fp64 (complex)
 void launch_dense_matvec(const cplx<double>* S, const cplx<double>* x, int P, double shift,

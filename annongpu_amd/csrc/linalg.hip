@@ -6,11 +6,14 @@
 // here S is a tiled GEMM with fp64 accumulation and the solve stays on the GPU.
 #include "kernels.hpp"
 
+#include <algorithm>
+
 namespace ann {
 
 namespace {
 
 constexpr int kRed = 1024;
+constexpr int kCus = 256;   // compute units of an MI355X
 
 __global__ __launch_bounds__(kRed) void weighted_sums_kernel(const cplx<double>* e, const double* w,
                                                              int64_t n, double* out) {
@@ -126,13 +129,17 @@ __device__ inline int64_t xcd_tile(int64_t b, int64_t n) {
 // ------------------------------------------------------------------ Gram
 // S[k][k'] = sum_s w_s conj(O_sk) O_sk' for the upper-triangular tile pairs, mirrored
 // into the lower triangle; samples are the k of the product, 16 per stage, staged in
-// LDS double-buffered with the next stage's global loads in flight during the MFMAs.
+// LDS double-buffered with the next stage's global loads in flight during the MFMAs.  With
+// part, workgroup (tile, z) takes the samples of chunk z and leaves its tile there
+// ([chunk][tile][64][64]) for gram_finish_kernel.
 template <typename T>
-__global__ __launch_bounds__(256) void gram_mfma_kernel(const cplx<T>* O, const double* w, int64_t count, int P,
-                                                        int64_t pairs, cplx<double>* S) {
+__global__ __launch_bounds__(256) void gram_mfma_kernel(const cplx<T>* O, const double* w, int64_t total, int P,
+                                                        int64_t pairs, int64_t chunk, cplx<double>* part,
+                                                        cplx<double>* S) {
     extern __shared__ double lds[];   // [2][kCStage]
     const int64_t t = xcd_tile(blockIdx.x, pairs);
     if (t >= pairs) return;
+    const int64_t first = int64_t(blockIdx.y) * chunk, count = first + chunk < total ? first + chunk : total;
     int ti, tj;
     upper_pair(t, ti, tj);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -164,12 +171,12 @@ __global__ __launch_bounds__(256) void gram_mfma_kernel(const cplx<T>* O, const 
     };
     CTileAcc acc;
     ctile_zero(acc);
-    const int64_t stages = (count + kCS - 1) / kCS;
-    fetch(0);
+    const int64_t stages = (count - first + kCS - 1) / kCS;
+    fetch(first);
     stash(lds);
     __syncthreads();
     for (int64_t g = 0; g < stages; g++) {
-        if (g + 1 < stages) fetch((g + 1) * kCS);
+        if (g + 1 < stages) fetch(first + (g + 1) * kCS);
         ctile_stage(lds + (g & 1) * kCStage, lane, wr, wc, acc);
         if (g + 1 < stages) stash(lds + ((g + 1) & 1) * kCStage);
         __syncthreads();
@@ -180,12 +187,33 @@ __global__ __launch_bounds__(256) void gram_mfma_kernel(const cplx<T>* O, const 
         for (int u = 0; u < 2; u++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int gr = row0 + ctile_row(lane, wr, tt, r), gc = col0 + ctile_col(lane, wc, u);
+                const int lr = ctile_row(lane, wr, tt, r), lc2 = ctile_col(lane, wc, u);
+                if (part) {
+                    part[((int64_t(blockIdx.y) * pairs + t) * kCT + lr) * kCT + lc2] = {acc.re[tt][u][r],
+                                                                                        acc.im[tt][u][r]};
+                    continue;
+                }
+                const int gr = row0 + lr, gc = col0 + lc2;
                 if (gr < P && gc < P) {
                     S[int64_t(gr) * P + gc] = {acc.re[tt][u][r], acc.im[tt][u][r]};
                     if (ti != tj) S[int64_t(gc) * P + gr] = {acc.re[tt][u][r], -acc.im[tt][u][r]};
                 }
             }
+}
+
+// the chunks' tiles added in chunk order, and the mirrored triangle
+__global__ __launch_bounds__(256) void gram_finish_kernel(const cplx<double>* part, int chunks, int P, int64_t pairs,
+                                                          cplx<double>* S) {
+    const int64_t t = blockIdx.x / (kCT * kCT / 256);
+    const int e = int(blockIdx.x % (kCT * kCT / 256)) * 256 + threadIdx.x;
+    int ti, tj;
+    upper_pair(t, ti, tj);
+    const int gr = ti * kCT + e / kCT, gc = tj * kCT + e % kCT;
+    if (gr >= P || gc >= P) return;
+    cplx<double> x = {0.0, 0.0};
+    for (int z = 0; z < chunks; z++) x = cadd(x, part[(int64_t(z) * pairs + t) * kCT * kCT + e]);
+    S[int64_t(gr) * P + gc] = x;
+    if (ti != tj) S[int64_t(gc) * P + gr] = cconj(x);
 }
 
 __global__ __launch_bounds__(256) void dense_matvec_kernel(const cplx<double>* S, const cplx<double>* x,
@@ -226,7 +254,6 @@ constexpr int kNB = 64;           // factor block
 // A small one is bound by its chain of launches and skips the second level.
 constexpr int kOuter = 256;
 constexpr int kOuterFrom = 2048;
-constexpr int kCus = 256;         // compute units of an MI355X
 
 // Scaled copy of the lower triangle: A[i][j] = (S + shift)[i][j] dinv_i dinv_j, j <= i,
 // dinv_i = (S_ii + shift)^-1/2 (1 where that is not positive), and row P = (dinv F)^H.
@@ -556,19 +583,47 @@ void launch_weighted_sums(const cplx<double>* e_loc, const double* w, int64_t co
     ANN_LAUNCH_CHECK();
 }
 
+// Sample chunks of the Gram: one where the tile pairs fill the chip, else chunks of whole
+// stages up to about two workgroups per CU, of at least 128 samples (below that the chunks'
+// tiles cost more traffic than the samples).  P = 648, 4,096 samples: 66 tiles on 256 CUs
+// 724 us, in 7 chunks 207 us with the reduction.
+static int gram_chunks(int P, int64_t count, int64_t* chunk) {
+    const int64_t nt = (P + kCT - 1) / kCT, pairs = nt * (nt + 1) / 2;
+    const int64_t want = std::max<int64_t>(1, std::min<int64_t>(2 * kCus / pairs, count / 128));
+    *chunk = std::max<int64_t>(kCS, ((count + want - 1) / want + kCS - 1) / kCS * kCS);
+    return int(std::max<int64_t>(1, (count + *chunk - 1) / *chunk));
+}
+
+size_t gram_work_elems(int P, int64_t count) {
+    int64_t chunk = 0;
+    const int z = gram_chunks(P, count, &chunk);
+    const int64_t nt = (P + kCT - 1) / kCT;
+    return z > 1 ? size_t(z) * (nt * (nt + 1) / 2) * kCT * kCT : 0;
+}
+
 template <typename T>
-void launch_gram(const cplx<T>* O, const double* w, int64_t count, int P, cplx<double>* S, hipStream_t stream) {
+void launch_gram(const cplx<T>* O, const double* w, int64_t count, int P, cplx<double>* work, cplx<double>* S,
+                 hipStream_t stream) {
     const int64_t nt = (P + kCT - 1) / kCT;
     const int64_t pairs = nt * (nt + 1) / 2;
     const size_t lds_bytes = sizeof(double) * 2 * kCStage;   // 64 KiB
     ANN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(gram_mfma_kernel<T>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(lds_bytes)));
     const int64_t grid = (pairs + 7) / 8 * 8;
-    gram_mfma_kernel<T><<<unsigned(grid), 256, lds_bytes, stream>>>(O, w, count, P, pairs, S);
+    int64_t chunk = 0;
+    const int chunks = gram_chunks(P, count, &chunk);
+    gram_mfma_kernel<T><<<dim3(unsigned(grid), unsigned(chunks)), 256, lds_bytes, stream>>>(
+        O, w, count, P, pairs, chunk, chunks > 1 ? work : nullptr, S);
     ANN_LAUNCH_CHECK();
+    if (chunks > 1) {
+        gram_finish_kernel<<<unsigned(pairs * (kCT * kCT / 256)), 256, 0, stream>>>(work, chunks, P, pairs, S);
+        ANN_LAUNCH_CHECK();
+    }
 }
-template void launch_gram<float>(const cplx<float>*, const double*, int64_t, int, cplx<double>*, hipStream_t);
-template void launch_gram<double>(const cplx<double>*, const double*, int64_t, int, cplx<double>*, hipStream_t);
+template void launch_gram<float>(const cplx<float>*, const double*, int64_t, int, cplx<double>*, cplx<double>*,
+                                 hipStream_t);
+template void launch_gram<double>(const cplx<double>*, const double*, int64_t, int, cplx<double>*, cplx<double>*,
+                                  hipStream_t);
 
 void launch_dense_matvec(const cplx<double>* S, const cplx<double>* x, int P, double shift, cplx<double>* y,
                          hipStream_t stream) {

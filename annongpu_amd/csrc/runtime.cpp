@@ -1277,22 +1277,42 @@ void tdvp_eval_t(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with_S) {
     t.has_samples = true;
     t.has_S = false;
     if (with_S) {
-        DevBuf<cplx<T>> O;
-        O.ensure(size_t(n) * P);
-        {
-            ScopedTimer timer("o_k");
-            launch_materialize_ok<T>(net, s.confs.p, s.words, g.p, n, t.Obar.p, O.p, S());
-        }
         t.S.ensure(size_t(P) * P);
-        {
+        // From the pairs of sites and pairs of units when nearly every (site, unit), the
+        // biases' constants included, carries a parameter: (N+1)^2 (M+1)^2 flop per sample
+        // against 4 P^2 for the Gram of the materialised O.  (They cross at a quarter of the
+        // pairs' count; the line is at a third, as the pairs' table has to be gathered.)
+        const double pairs = double(psi.N + 1) * (psi.M + 1);
+        if (pairs * pairs <= 3.0 * double(P) * P) {
+            const SpinPlan plan = spin_plan(net.N, net.M, net.Mpad, n, true);
+            if (!t.bits_valid) {
+                t.spin_bits.ensure(size_t(plan.bit_blocks) * plan.vpad);
+                launch_spin_bits(s.confs.p, s.words, n, net.N, plan.vpad, t.spin_bits.p, S());
+                t.bits_valid = true;
+            }
+            t.gram_work.ensure(dense_gram_work_elems(psi.N, psi.M, n));
+            t.gram_mean.ensure(P);
             ScopedTimer timer("gram");
-            launch_gram<T>(O.p, s.w.p, n, P, t.S.p, S());
+            launch_dense_gram<T>(psi.layout, psi.N, psi.M, psi.Mpad, psi.kind == PSI_DEEP ? t.conn.p : nullptr,
+                                 t.spin_bits.p, plan.vpad, g.p, s.w.p, n, P, t.gram_work.p, t.gram_mean.p, t.S.p, S());
+        } else {
+            DevBuf<cplx<T>> O;
+            O.ensure(size_t(n) * P);
+            {
+                ScopedTimer timer("o_k");
+                launch_materialize_ok<T>(net, s.confs.p, s.words, g.p, n, t.Obar.p, O.p, S());
+            }
+            t.gram_part.ensure(gram_work_elems(P, n));
+            {
+                ScopedTimer timer("gram");
+                launch_gram<T>(O.p, s.w.p, n, P, t.gram_part.p, t.S.p, S());
+            }
+            // reference S = sum w conj(O) O - conj(<O>) <O>; with centred O this needs
+            // (1 - sum w) conj(<O>) <O> added back (zero for normalised weights)
+            t.settle();
+            if (std::abs(1.0 - t.wsum) > 0.0) launch_rank1(t.S.p, t.Obar.p, P, 1.0 - t.wsum, S());
+            Runtime::get().sync();
         }
-        // reference S = sum w conj(O) O - conj(<O>) <O>; with centred O this needs
-        // (1 - sum w) conj(<O>) <O> added back (zero for normalised weights)
-        t.settle();
-        if (std::abs(1.0 - t.wsum) > 0.0) launch_rank1(t.S.p, t.Obar.p, P, 1.0 - t.wsum, S());
-        Runtime::get().sync();
         t.has_S = true;
     }
 }
@@ -1380,9 +1400,10 @@ void tdvp_eval_generic(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with
     t.has_S = false;
     if (with_S) {
         t.S.ensure(size_t(P) * P);
+        t.gram_part.ensure(gram_work_elems(P, n));
         {
             ScopedTimer timer("gram");
-            launch_gram<T>(O.p, s.w.p, n, P, t.S.p, S());
+            launch_gram<T>(O.p, s.w.p, n, P, t.gram_part.p, t.S.p, S());
         }
         // S = sum w conj(O) O - conj(<O>) <O>
         launch_rank1(t.S.p, t.Obar.p, P, -1.0, S());

@@ -396,6 +396,9 @@ struct Tdvp {
     DevBuf<cplx<double>> S, Obar, Fd;
     DevBuf<cplx<double>> chol, chol_work;   // Cholesky factor of the scaled S + shift and its panel workspace
     DevBuf<double> chol_dinv;               // the diagonal scaling of that factor
+    DevBuf<double> gram_work;               // pair products of a dense net's S (gram_dense.hip)
+    DevBuf<cplx<double>> gram_mean;
+    DevBuf<cplx<double>> gram_part;         // sample chunks of the Gram of a materialised O
     // structured O of the last evaluation (dense nets)
     int precision = 0, words = 0, N = 0, M = 0, Mpad = 0, C = 0, layout = 0, npad = 0;
     int64_t count = 0;

@@ -1,0 +1,68 @@
+"""S of a one-layer net from pairs of sites and units against the Gram of its O_k samples, at the
+edges of the kernel's tiles (64 site pairs a wave, 32 unit pairs, 16 samples a stage, 64-sample
+words) and over the layouts that reach it, sample counts and weights that do not sum to one.
+
+The O_k samples are exact copies of what S is built from, so both sides are fp64 sums of the
+same products: |S - S_ref| <= 4 n eps max|sum w |O_k|^2| entrywise (n summands)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def net(kind, N, M, rng):
+    import annongpu_amd as A
+
+    def gauss(shape, sigma):
+        return sigma * (rng.standard_normal(shape) + 1j * rng.standard_normal(shape))
+
+    if kind == "rbm":
+        return A.PsiRBM(gauss((N, M), 0.2), final_weight=1.5 - 0.5j)
+    if kind == "circulant":
+        conn = (np.arange(M)[None, :] + np.arange(N)[:, None]) % N
+    elif kind == "shuffled":
+        conn = np.stack([rng.permutation(N) for _ in range(M)], axis=1)
+    else:   # repeated: every unit reads one of its sites twice
+        conn = np.stack([np.concatenate([rng.permutation(N), rng.integers(0, N, 1)]) for _ in range(M)], axis=1)
+    return A.PsiDeep(N, gauss(N, 0.1), [gauss(M, 0.1)], [conn], [gauss(conn.shape, 0.2)], 1.0 + rng.random(M))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("kind,N,M,n", [("circulant", 1, 1, 1), ("circulant", 11, 6, 65), ("rbm", 11, 7, 64),
+                                        ("rbm", 12, 24, 1000), ("shuffled", 23, 9, 129), ("circulant", 22, 8, 15),
+                                        ("repeated", 16, 5, 300), ("circulant", 70, 3, 63)])
+def test_dense_gram(kind, N, M, n, precision):
+    import annongpu_amd as A
+    rng = np.random.default_rng(100 * N + M)
+    psi = net(kind, N, M, rng)
+    psi.precision = precision
+    words = (N + 63) // 64
+    confs = rng.integers(0, 2 ** 63, size=(n, words), dtype=np.uint64)
+    if N % 64:
+        confs[:, -1] &= np.uint64(2 ** (N % 64) - 1)
+    w = rng.random(n) / n
+    t = A.TDVP(psi.num_params)
+    t.eval(A.Operator(1.0 * A.sigma_z(0)), psi, A.SampleList(N, confs, w))
+    O = t.O_k_samples
+    mean = w @ O
+    S = (O.conj() * w[:, None]).T @ O - np.outer(mean.conj(), mean)
+    assert np.abs(t.S_matrix - S).max() <= 4 * max(n, 8) * np.finfo(float).eps * (w @ np.abs(O) ** 2).max()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [1, 127, 129, 300, 1025])
+def test_gram_of_materialised_samples(n, precision):
+    """S of a PsiCNN (no pair structure) at the edges of the Gram's sample chunks: the fp64 rank-one
+    term and n summands, entrywise as above."""
+    import annongpu_amd as A
+    rng = np.random.default_rng(n)
+    psi = A.seeded_cnn([1, 3, 4], [(3, [1, 2, 2]), (2, [1, 3, 2])], seed=n, sigma=0.2)
+    psi.precision = precision
+    confs = rng.integers(0, 2 ** 12, size=(n, 1), dtype=np.uint64)
+    w = rng.random(n) / n
+    t = A.TDVP(psi.num_params)
+    t.eval(A.Operator(1.0 * A.sigma_z(0)), psi, A.SampleList(12, confs, w))
+    O = t.O_k_samples
+    mean = w @ O
+    S = (O.conj() * w[:, None]).T @ O - np.outer(mean.conj(), mean)
+    assert np.abs(t.S_matrix - S).max() <= 4 * max(n, 8) * np.finfo(float).eps * (w @ np.abs(O) ** 2).max()
