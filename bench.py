@@ -295,7 +295,9 @@ def dense_S_leg(A, steps=2, warmup=1):
     ms = (time.perf_counter() - t0) / steps * 1e3
     g_ms, g_n = A.profiler_query("gram")
     c_ms, c_n = A.profiler_query("cholesky")
-    gram_flop = 4.0 * B * P * P            # upper-triangular half of the Hermitian O^H W O (real flops)
+    # S from pairs of sites (real) and pairs of units (complex, Hermitian), the constants of the
+    # biases included: 4 real flops per sample and pair of pairs
+    gram_flop = 4.0 * B * (1 + N * (N + 1) / 2) * ((M + 1) * (M + 2) / 2)
     chol_flop = 4.0 / 3.0 * P ** 3         # complex Cholesky (real flops); the two triangular solves excluded
     g_avg, c_avg = g_ms / max(g_n, 1), c_ms / max(c_n, 1)
     return {"workload": "Heisenberg ring N=64 PBC, PsiDeep M=256 (P=16,704), 8192 persistent exchange chains, "
