@@ -308,7 +308,8 @@ __global__ __launch_bounds__(kBlock) void mc_sweep_kernel(DenseView<T> net, uint
     }
 }
 
-// E_loc(s) = sum_groups coef_g(s) * psi(s')/psi(s)  (Operator.hpp:36-121)
+// E_loc(s) = sum_groups coef_g(s) * psi(s')/psi(s)  (Operator.hpp:36-121), any strings (in
+// fp32 those that flip at most two sites are served by eloc_dense.hip)
 template <typename T, int U>
 __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? 4 : 1) void local_energy_kernel(DenseView<T> net, OpView op,
                                                               const uint64_t* confs,
@@ -820,6 +821,12 @@ template <typename T>
 void launch_local_energy(const DenseView<T>& net, const OpView& op, const uint64_t* confs,
                          const cplx<T>* theta, int64_t count, cplx<double>* e_loc, hipStream_t stream) {
     if (count <= 0) return;
+    if constexpr (sizeof(T) == 4) {
+        if (local_energy_terms_supported(op)) {
+            launch_local_energy_terms(net, op, confs, theta, count, e_loc, stream);
+            return;
+        }
+    }
     dispatch_u(net.Mpad / 64, [&](auto tag) {
         constexpr int U = std::decay_t<decltype(tag)>::value;
         local_energy_kernel<T, U><<<grid_waves(count), kBlock, 0, stream>>>(net, op, confs, theta, count,

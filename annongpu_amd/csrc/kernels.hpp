@@ -70,6 +70,10 @@ struct OpView {
     const int* group_begin;          // [num_groups + 1] ranges into the string arrays
     const uint64_t* string_zy;       // [num_strings][words]  Z|Y mask (b bits)
     const double* string_coef;       // [num_strings][2] coefficient * (-i)^{#Y}
+    const int* group_sites;          // [num_groups][2] the flipped sites of a group of one or two (-1: none)
+    int diag_group;                  // the group without flips (-1: none)
+    int max_flips;                   // most sites any group flips
+    int equal_spins;                 // a group of two sites may have a coefficient where their spins are equal
 };
 
 // Pauli-sum operator acting on Pauli-string configurations (string n maps x to
@@ -118,6 +122,11 @@ template <typename T>
 void launch_mc_sweep(const DenseView<T>& net, uint64_t* chain_confs, cplx<T>* theta, int num_chains,
                      int words, int move, int64_t num_proposals, uint64_t counter, uint64_t seed,
                      uint32_t* accepted, hipStream_t stream);
+
+// E_loc of the operators local_energy_terms_supported accepts, fp32 (eloc_dense.hip)
+bool local_energy_terms_supported(const OpView& op);
+void launch_local_energy_terms(const DenseView<float>& net, const OpView& op, const uint64_t* confs,
+                               const cplx<float>* theta, int64_t count, cplx<double>* e_loc, hipStream_t stream);
 
 template <typename T>
 void launch_local_energy(const DenseView<T>& net, const OpView& op, const uint64_t* confs,

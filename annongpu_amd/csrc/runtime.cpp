@@ -703,6 +703,37 @@ const DeviceOp& Operator::device(int words) {
     }
     begin.push_back(int(scoef.size() / 2));
     d->num_groups = int(groups.size());
+    std::vector<int> sites;   // the flipped sites of every group of at most two
+    for (size_t g = 0; g < groups.size(); g++) {
+        int n = 0, at[2] = {-1, -1};
+        for (int w = 0; w < words; w++)
+            for (uint64_t m = masks[g][w]; m; m &= m - 1, n++)
+                if (n < 2) at[n] = 64 * w + __builtin_ctzll(m);
+        sites.insert(sites.end(), at, at + 2);
+        d->max_flips = std::max(d->max_flips, n);
+        if (n == 0) d->diag_group = int(g);
+    }
+    d->group_sites.upload(sites.data(), sites.size());
+    // Groups of two sites whose strings read no other site: their coefficient where the two
+    // spins are equal (a bond's X X + Y Y has none); strings that read others may have one.
+    for (size_t g = 0; g < groups.size(); g++) {
+        if (sites[2 * g + 1] < 0) continue;
+        cd up = 0.0, down = 0.0;
+        for (int n : groups[g]) {
+            int ny = 0, nb = 0;
+            for (int w = 0; w < kMaxWords; w++) {
+                const uint64_t aw = a[size_t(n) * kMaxWords + w], bw = b[size_t(n) * kMaxWords + w];
+                const uint64_t m = w < words ? masks[g][w] : 0;
+                if (bw & ~m) d->equal_spins = true;
+                ny += __builtin_popcountll(~aw & bw);
+                nb += __builtin_popcountll(bw);
+            }
+            static const cd phase[4] = {cd(1, 0), cd(0, -1), cd(-1, 0), cd(0, 1)};
+            up += coef[n] * phase[ny & 3];
+            down += coef[n] * phase[ny & 3] * (nb & 1 ? -1.0 : 1.0);
+        }
+        if (up != 0.0 || down != 0.0) d->equal_spins = true;
+    }
     d->group_flip.upload(flip.data(), flip.size());
     d->group_begin.upload(begin.data(), begin.size());
     d->string_zy.upload(zy.data(), zy.size());

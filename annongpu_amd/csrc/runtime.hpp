@@ -279,10 +279,13 @@ struct DeviceOp {
     int words = 0;
     int num_groups = 0;
     DevBuf<uint64_t> group_flip, string_zy;
-    DevBuf<int> group_begin;
+    DevBuf<int> group_begin, group_sites;
+    int diag_group = -1, max_flips = 0;
+    bool equal_spins = false;
     DevBuf<double> string_coef;
     OpView view() const {
-        return {num_groups, words, group_flip.p, group_begin.p, string_zy.p, string_coef.p};
+        return {num_groups, words, group_flip.p, group_begin.p, string_zy.p, string_coef.p, group_sites.p, diag_group,
+                max_flips, equal_spins ? 1 : 0};
     }
 };
 
