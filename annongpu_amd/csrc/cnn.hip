@@ -1021,9 +1021,12 @@ __global__ __launch_bounds__(64) void classical_ok_kernel(ClassicalView<T, R> v,
 }
 
 // kernels with more than 64 KiB of LDS per block must opt in (at most the 160 KiB of a gfx950 CU)
+inline void check_lds(size_t bytes) {
+    if (bytes > 160 * 1024) throw std::invalid_argument("the network state of one configuration exceeds the 160 KiB LDS of a CU");
+}
 template <typename K>
 void allow_lds(K kernel, size_t bytes) {
-    if (bytes > 160 * 1024) throw std::invalid_argument("the network state of one configuration exceeds the 160 KiB LDS of a CU");
+    check_lds(bytes);
     if (bytes > 64 * 1024)
         ANN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
@@ -1175,6 +1178,9 @@ template <typename V>
 void launch_generic_log_psi(const V& net, const uint64_t* confs, int words, int64_t count,
                             cplx<double> log_prefactor, cplx<double>* log_psi, double* weight, hipStream_t stream) {
     if (count <= 0) return;
+    check_lds(forward_lds(net));
+    if constexpr (std::is_same<V, CnnView<typename V::real_t>>::value)
+        if (cnn_pair_log_psi(net, confs, words, count, log_prefactor, log_psi, weight, stream)) return;
     allow_lds(generic_log_psi_kernel<V>, forward_lds(net));
     generic_log_psi_kernel<V><<<grid_for(count), 64, forward_lds(net), stream>>>(net, confs, words, count,
                                                                                  log_prefactor, log_psi, weight);
@@ -1188,6 +1194,9 @@ void launch_generic_mc(const V& net, uint64_t* chain_confs, int words, int num_c
     if (num_chains <= 0 || num_proposals <= 0) return;
     using T = typename V::real_t;
     if constexpr (std::is_same<V, CnnView<T>>::value) {
+        // (a net is refused by its size alone, whatever kernels serve it)
+        check_lds(cnn_inc_lds(net) + cnn_stage_bytes(net));
+        if (cnn_pair_mc(net, chain_confs, words, num_chains, move, num_proposals, counter, seed, accepted, stream)) return;
         const int stage = cnn_stage_bytes(net);
         dispatch_vmax(net, [&](auto vt) {
             constexpr int VM = decltype(vt)::value;
@@ -1217,6 +1226,8 @@ void launch_generic_local_energy(const V& net, const OpView& op, const uint64_t*
     if (count <= 0) return;
     using T = typename V::real_t;
     if constexpr (std::is_same<V, CnnView<T>>::value) {
+        check_lds(cnn_inc_lds(net) + cnn_stage_bytes(net));
+        if (cnn_pair_local_energy(net, op, confs, count, e_loc, stream)) return;
         const int stage = cnn_stage_bytes(net);
         dispatch_vmax(net, [&](auto vt) {
             constexpr int VM = decltype(vt)::value;
@@ -1243,6 +1254,8 @@ void launch_generic_ok(const V& net, const uint64_t* confs, int words, int64_t c
     if (count <= 0) return;
     using T = typename V::real_t;
     if constexpr (std::is_same<V, CnnView<T>>::value) {
+        check_lds(ok_lds(net));
+        if (!center && cnn_pair_ok(net, confs, words, count, O, stream)) return;
         allow_lds(cnn_ok_kernel<T>, ok_lds(net));
         cnn_ok_kernel<T><<<grid_for(count), 64, ok_lds(net), stream>>>(net, confs, words, count, center, O);
     } else if constexpr (std::is_same<V, MlpView<T>>::value) {

@@ -9,6 +9,24 @@ namespace ann {
 
 constexpr int kMaxCnnLayers = 3;
 
+// Tables of a two-layer PsiCNN of one symmetry class whose first kernel has at most nine sites
+// (cnn_pair.hip); wf is null for other nets.  wf, wb: the second layer's weights, output (wf) or
+// input (wb) channels in blocks of cb, padded with zeros: wf[block][ci][k][cb], wb[block][cj][k][cb].
+template <typename T>
+struct CnnPair {
+    int N, C0, C1, v0, v1;
+    int n0, n1;              // sites that read a given site in layer 0, and that a flip reaches in layer 1
+    int cb, blocks, blocks0;
+    int self0;               // the kernel site of layer 0 that is the site itself
+    const cplx<T>* wf;
+    const cplx<T>* wb;
+    const uint32_t* aff0;    // [N][n0] reading site | bits of its pattern << 8
+    const uint8_t* aff1;     // [N][n1] reached sites in increasing order
+    const uint64_t* mask1;   // [N][kMaxWords] the same as masks
+    const int* nbr1;         // [N][v1] neighbour table of layer 1
+    const uint8_t* inv1;     // [N][v1] the site whose neighbour k is the given one
+};
+
 // PsiCNN in dim 3 (include/quantum_state/PsiCNN.hpp:32-87).  Parameter k of
 // link (layer l, input channel ci, output channel cj), symmetry class c and
 // kernel offset o sits at link_off[l] + ((ci * ch[l] + cj) * nsym + c) * vol[l] + o
@@ -35,6 +53,7 @@ struct CnnView {
     // cons[(l * N + y) * kMaxWords + k]: word k of the mask of the sites x whose layer-l
     // pre-activations read site y (the consumers of y, for the local updates)
     const uint64_t* cons;
+    CnnPair<T> pair;
 };
 
 constexpr int kMaxMlpLayers = 4;
@@ -99,6 +118,20 @@ struct ClassicalView {
     R ref;                   // over N spins (a PsiDeep also over the 3 N units of a Pauli string)
     cplx<T> ref_lp;          // the reference's log_prefactor
 };
+
+// The kernels of cnn_pair.hip; false (and nothing launched) where they do not serve the net, the
+// move or the operator
+template <typename T>
+bool cnn_pair_log_psi(const CnnView<T>& v, const uint64_t* confs, int words, int64_t count, cplx<double> lp,
+                      cplx<double>* log_psi, double* weight, hipStream_t stream);
+template <typename T>
+bool cnn_pair_mc(const CnnView<T>& v, uint64_t* chain_confs, int words, int num_chains, int move, int64_t num_proposals,
+                 uint64_t counter, uint64_t seed, uint32_t* accepted, hipStream_t stream);
+template <typename T>
+bool cnn_pair_local_energy(const CnnView<T>& v, const OpView& op, const uint64_t* confs, int64_t count,
+                           cplx<double>* e_loc, hipStream_t stream);
+template <typename T>
+bool cnn_pair_ok(const CnnView<T>& v, const uint64_t* confs, int words, int64_t count, cplx<T>* O, hipStream_t stream);
 
 // Kernels of the wave functions without a structured O (V = CnnView<T> or MlpView<T>):
 // one 64-lane wavefront per configuration, a full forward pass per configuration,

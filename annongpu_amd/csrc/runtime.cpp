@@ -250,6 +250,83 @@ void Psi::upload_mlp_tables() {
     mlp_ri.upload(ri.data(), ri.size());
 }
 
+// neighbour tables (Convolve.hpp:122-148), consumer masks and symmetry classes of a PsiCNN, and
+// the tables of cnn_pair.hip where it serves the net
+void Psi::build_cnn_tables() {
+    const int e0 = extent[0], e1 = extent[1], e2 = extent[2], page = e1 * e2;
+    std::vector<int> nbr;
+    for (int l = 0; l < cnn_layers; l++) {
+        const int* cv = &connectivity[3 * l];
+        for (int x = 0; x < N; x++) {
+            const int pg = x / page, row = (x % page) / e2, col = x % e2;
+            for (int k = 0; k < cv[0]; k++)
+                for (int i = 0; i < cv[1]; i++)
+                    for (int j = 0; j < cv[2]; j++)
+                        nbr.push_back(((pg + k) % e0) * page + ((row + i) % e1) * e2 + (col + j) % e2);
+        }
+    }
+    nbr_d.upload(nbr.data(), nbr.size());
+    // consumers of every site in every layer (the receptive fields of the local updates)
+    std::vector<uint64_t> cons(size_t(cnn_layers) * N * kMaxWords, 0);
+    std::vector<int> vol(cnn_layers);
+    size_t off = 0;
+    for (int l = 0; l < cnn_layers; l++) {
+        const int* cv = &connectivity[3 * l];
+        vol[l] = cv[0] * cv[1] * cv[2];
+        for (int x = 0; x < N; x++)
+            for (int k = 0; k < vol[l]; k++) {
+                const int y = nbr[off + size_t(x) * vol[l] + k];
+                cons[(size_t(l) * N + y) * kMaxWords + (x >> 6)] |= uint64_t(1) << (x & 63);
+            }
+        off += size_t(N) * vol[l];
+    }
+    cons_d.upload(cons.data(), cons.size());
+    sym_d.upload(sym.data(), sym.size());
+    cnn_tables = true;
+    pair = {};
+    if (cnn_layers != 2 || num_sym != 1 || vol[0] > 9 || vol[1] > 9 || N > 64 * kMaxWords) return;
+    auto sites = [&](const uint64_t* m) {
+        std::vector<int> v;
+        for (int x = 0; x < N; x++)
+            if ((m[x >> 6] >> (x & 63)) & 1) v.push_back(x);
+        return v;
+    };
+    const int v0 = vol[0], v1 = vol[1];
+    std::vector<uint32_t> aff0;
+    std::vector<uint8_t> aff1, inv1(size_t(N) * v1);
+    std::vector<uint64_t> mask1(size_t(N) * kMaxWords, 0);
+    for (int i = 0; i < N; i++) {
+        const auto first = sites(&cons[size_t(i) * kMaxWords]);
+        for (int y : first) {
+            uint32_t bits = 0;
+            for (int k = 0; k < v0; k++) bits |= uint32_t(nbr[size_t(y) * v0 + k] == i) << k;
+            aff0.push_back(uint32_t(y) | bits << 8);
+            for (int q = 0; q < kMaxWords; q++) mask1[size_t(i) * kMaxWords + q] |= cons[(size_t(N) + y) * kMaxWords + q];
+        }
+        const auto reach = sites(&mask1[size_t(i) * kMaxWords]);
+        // the lattice is periodic: every site is read by as many sites
+        if (i > 0 && (int(first.size()) != pair.n0 || int(reach.size()) != pair.n1)) return;
+        pair.n0 = int(first.size());
+        pair.n1 = int(reach.size());
+        aff1.insert(aff1.end(), reach.begin(), reach.end());
+    }
+    for (int x = 0; x < N; x++)
+        for (int k = 0; k < v1; k++) inv1[size_t(nbr[size_t(N) * v0 + size_t(x) * v1 + k]) * v1 + k] = uint8_t(x);
+    pair_aff0.upload(aff0.data(), aff0.size());
+    pair_aff1.upload(aff1.data(), aff1.size());
+    pair_inv1.upload(inv1.data(), inv1.size());
+    pair_mask1.upload(mask1.data(), mask1.size());
+    pair.N = N;
+    pair.C0 = channels[0];
+    pair.C1 = channels[1];
+    pair.v0 = v0;
+    pair.v1 = v1;
+    const int most = std::max(pair.C0, pair.C1);
+    pair.cb = most <= 2 ? 2 : most <= 4 ? 4 : 8;
+    pair.blocks = (pair.C1 + pair.cb - 1) / pair.cb;
+    pair.blocks0 = (pair.C0 + pair.cb - 1) / pair.cb;
+}
+
 void Psi::sync_device() {
     if (!dirty && params_dirty) {
         // parameters only: one asynchronous copy and a repack on the device
@@ -265,39 +342,24 @@ void Psi::sync_device() {
     if (!dirty) return;
     params_dirty = false;
     if (kind == PSI_CNN) {
-        // parameters, neighbour tables (Convolve.hpp:122-148) and symmetry classes
-        cp64.upload(reinterpret_cast<const cplx<double>*>(params.data()), params.size());
-        std::vector<cplx<float>> p32(params.size());
-        for (size_t i = 0; i < params.size(); i++) p32[i] = {float(params[i].real()), float(params[i].imag())};
-        cp32.upload(p32.data(), p32.size());
-        const int e0 = extent[0], e1 = extent[1], e2 = extent[2], page = e1 * e2;
-        std::vector<int> nbr;
-        for (int l = 0; l < cnn_layers; l++) {
-            const int* cv = &connectivity[3 * l];
-            for (int x = 0; x < N; x++) {
-                const int pg = x / page, row = (x % page) / e2, col = x % e2;
-                for (int k = 0; k < cv[0]; k++)
-                    for (int i = 0; i < cv[1]; i++)
-                        for (int j = 0; j < cv[2]; j++)
-                            nbr.push_back(((pg + k) % e0) * page + ((row + i) % e1) * e2 + (col + j) % e2);
-            }
+        // the tables of the structure once, then the parameters and, for cnn_pair.hip, the
+        // second layer's weights in channel blocks behind them
+        if (!cnn_tables) build_cnn_tables();
+        std::vector<cd> p(params);
+        if (pair.cb) {
+            const int C0 = pair.C0, C1 = pair.C1, v = pair.v1, cb = pair.cb;
+            const size_t w0 = size_t(C0) * pair.v0, f0 = p.size();
+            p.resize(f0 + size_t(pair.blocks) * C0 * v * cb + size_t(pair.blocks0) * C1 * v * cb, 0.0);
+            const size_t b0 = f0 + size_t(pair.blocks) * C0 * v * cb;
+            for (int ci = 0; ci < C0; ci++)
+                for (int cj = 0; cj < C1; cj++)
+                    for (int k = 0; k < v; k++) {
+                        const cd x = params[w0 + (size_t(ci) * C1 + cj) * v + k];
+                        p[f0 + ((size_t(cj / cb) * C0 + ci) * v + k) * cb + cj % cb] = x;
+                        p[b0 + ((size_t(ci / cb) * C1 + cj) * v + k) * cb + ci % cb] = x;
+                    }
         }
-        nbr_d.upload(nbr.data(), nbr.size());
-        // consumers of every site in every layer (the receptive fields of the local updates)
-        std::vector<uint64_t> cons(size_t(cnn_layers) * N * kMaxWords, 0);
-        size_t off = 0;
-        for (int l = 0; l < cnn_layers; l++) {
-            const int* cv = &connectivity[3 * l];
-            const int vol = cv[0] * cv[1] * cv[2];
-            for (int x = 0; x < N; x++)
-                for (int k = 0; k < vol; k++) {
-                    const int y = nbr[off + size_t(x) * vol + k];
-                    cons[(size_t(l) * N + y) * kMaxWords + (x >> 6)] |= uint64_t(1) << (x & 63);
-                }
-            off += size_t(N) * vol;
-        }
-        cons_d.upload(cons.data(), cons.size());
-        sym_d.upload(sym.data(), sym.size());
+        up_both(cp64, cp32, p);
         dirty = false;
         return;
     }
@@ -430,6 +492,13 @@ static CnnView<T> make_cnn_view(const Psi& q, const cplx<T>* p, const int* nbr, 
     v.nbr = nbr;
     v.sym = sym;
     v.cons = q.cons_d.p;
+    if (q.pair.cb) {
+        const CnnPair<double>& s = q.pair;
+        const cplx<T>* wf = p + q.num_params;
+        v.pair = {s.N,  s.C0, s.C1, s.v0, s.v1, s.n0, s.n1, s.cb, s.blocks, s.blocks0, 0,
+                  wf,   wf + size_t(s.blocks) * s.C0 * s.v1 * s.cb,
+                  q.pair_aff0.p, q.pair_aff1.p, q.pair_mask1.p, nbr + v.nbr_off[1], q.pair_inv1.p};
+    }
     return v;
 }
 

@@ -243,6 +243,12 @@ struct Psi {
     DevBuf<int> nbr_d;
     DevBuf<uint32_t> sym_d;
     DevBuf<uint64_t> cons_d;
+    bool cnn_tables = false;       // the structure's tables are on the device (they never change)
+    CnnPair<double> pair{};        // sizes of cnn_pair.hip's tables (cb = 0: not served)
+    DevBuf<uint32_t> pair_aff0;
+    DevBuf<uint8_t> pair_aff1, pair_inv1;
+    DevBuf<uint64_t> pair_mask1;
+    void build_cnn_tables();
     // multi-layer PsiDeep device state (layers concatenated; offsets per layer)
     DevBuf<uint32_t> mlp_cn;
     DevBuf<cplx<double>> mlp_w64, mlp_b64;
