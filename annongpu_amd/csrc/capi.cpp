@@ -944,7 +944,7 @@ int ann_local_energies_noalloc(ann_operator op, ann_psi psi, const uint64_t* con
         if (q.precision == 0) {
             auto v = q.view64();
             auto* t = static_cast<ann::cplx<double>*>(th);
-            ann::launch_theta_valu<double>(v, confs, q.words, count, t, st);
+            ann::launch_theta64(v, confs, q.words, count, t, st);
             ann::launch_local_energy<double>(v, d.view(), confs, t, count, out, st);
         } else {
             auto v = q.view32();

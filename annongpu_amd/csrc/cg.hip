@@ -80,12 +80,17 @@ __global__ __launch_bounds__(256) void cg_step_kernel(cplx<double>* x, cplx<doub
                                                       const cplx<double>* p, const cplx<double>* Ap,
                                                       const double* diag, double shift, int64_t n,
                                                       int64_t jac_end, const double* rzpart, int rz_parts,
-                                                      const double* apart, int a_parts, double* newpart,
+                                                      DotParts apart, double* newpart,
                                                       const int* done) {
     __shared__ double sh[4];
     if (done[0]) return;
     const double rz = total_rz(rzpart, rz_parts, sh);
-    const double pap = total(apart, a_parts, 2, 0, sh);
+    double pa = 0.0;
+    if (int(threadIdx.x) < apart.n) {
+        const double* q = apart.p + int64_t(threadIdx.x) * apart.stride;
+        pa = apart.stride == 2 ? q[0] : q[0] + q[1] + q[2] + q[3];
+    }
+    const double pap = block_sum(pa, sh);
     const double alpha = pap > 0.0 ? rz / pap : 0.0;
     double rz2 = 0.0, rr = 0.0;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256) {
@@ -199,11 +204,11 @@ void launch_pcg_pap(const cplx<double>* p, const cplx<double>* Ap, int64_t n, do
 
 void launch_pcg_step(cplx<double>* x, cplx<double>* r, cplx<double>* z, const cplx<double>* p,
                     const cplx<double>* Ap, const double* diag, double shift, int64_t n, int64_t jac_end,
-                    const double* rzpart, const double* apart, int a_parts, double* newpart, const int* done,
+                    const double* rzpart, const DotParts& apart, double* newpart, const int* done,
                     hipStream_t stream) {
-    if (a_parts > 256) throw std::invalid_argument("too many partial sums");
+    if (apart.n > 256) throw std::invalid_argument("too many partial sums");
     cg_step_kernel<<<kCgParts, 256, 0, stream>>>(x, r, z, p, Ap, diag, shift, n, jac_end, rzpart, kCgParts, apart,
-                                                 a_parts, newpart, done);
+                                                 newpart, done);
     ANN_LAUNCH_CHECK();
 }
 

@@ -47,24 +47,6 @@ __global__ void enumerate_paulis_kernel(uint64_t* confs, int64_t first, int64_t 
     confs[2 * i + 1] = b;
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void theta_valu_kernel(DenseView<T> net, const uint64_t* confs,
-                                                            int words, int64_t count, cplx<T>* theta) {
-    const int64_t s = blockIdx.x;
-    if (s >= count) return;
-    const Conf c = load_conf(confs, s, words);
-    for (int j = threadIdx.x; j < net.Mpad; j += blockDim.x) {
-        cplx<T> t = net.b[j];
-        for (int v = 0; v < net.N; v++) {
-            const cplx<T> w = net.Wd[int64_t(v) * net.Mpad + j];
-            const T sv = spin_bit(c, v) ? T(1) : T(-1);
-            t.re += sv * w.re;
-            t.im += sv * w.im;
-        }
-        theta[s * net.Mpad + j] = t;
-    }
-}
-
 // theta on MFMA.  One wavefront computes 16 samples x 64 real columns (4 tiles
 // of v_mfma_f32_16x16x16_bf16).  A fragment: lane l holds row l%16, k = 4(l/16)+0..3
 // (spins, exact in bf16); B fragment: k = 4(l/16)+0..3, column l%16 (pre-packed).
@@ -461,161 +443,6 @@ __global__ void materialize_ok_kernel(DenseView<T> net, const uint64_t* confs, i
     O[s * net.num_params + k] = o;
 }
 
-// Y[v][c] = sum_s spin_sv X_sc on fp64 MFMA (v_mfma_f64_16x16x4_f64), the
-// transpose-GEMM behind <O>, F, the gradient and the O^H u half of S.v for a
-// dense net.  Rows v < N are spins (+-1, exact), row N is all ones (bias
-// parameters).  Columns: X_s,2j / 2j+1 = re / im of coef_s * g_sj (or
-// conj g_sj), columns 2 Mpad / 2 Mpad+1 = re / im of coef_s (visible
-// parameters).  One wavefront owns one 16-column tile for up to 8 row tiles and a
-// chunk of samples; lane l feeds sample 4t + l/16 of step t (A: row l%16, B:
-// column l%16, both at k = l/16).  Partial tiles per
-// chunk are summed by sum_partials_kernel in a fixed order (deterministic).
-typedef double double4_t __attribute__((ext_vector_type(4)));
-constexpr int kRowTilesPerWave = 8;
-
-template <typename T>
-__global__ __launch_bounds__(64) void spin_gemm_kernel(DenseView<T> net, const uint64_t* confs, int words,
-                                                       const cplx<T>* g, int conj_g, const cplx<double>* coef,
-                                                       int64_t count, int64_t chunk, int vpad, int ncols,
-                                                       double* partial) {
-    const int lane = threadIdx.x;
-    const int col = blockIdx.x * 16 + (lane & 15);
-    const int kk = lane >> 4;
-    const int vt0 = blockIdx.z * kRowTilesPerWave;
-    const int vtiles = vpad / 16;
-    const int64_t s0 = int64_t(blockIdx.y) * chunk;
-    const int64_t s1 = s0 + chunk < count ? s0 + chunk : count;
-    const int two_m = 2 * net.Mpad;
-    const bool is_g = col < two_m;
-    const bool is_coef = col >= two_m && col < two_m + 2;
-    const int j = col >> 1;
-    const bool imag_part = col & 1;
-    double4_t acc[kRowTilesPerWave];
-#pragma unroll
-    for (int t = 0; t < kRowTilesPerWave; t++) acc[t] = {0.0, 0.0, 0.0, 0.0};
-    constexpr int kStage = 4;   // MFMA steps whose operands are loaded together
-    for (int64_t sq = s0; sq < s1; sq += 4 * kStage) {
-        double x[kStage];
-        uint64_t cw[kStage][kMaxWords];
-#pragma unroll
-        for (int st = 0; st < kStage; st++) {
-            const int64_t s = sq + 4 * st + kk;
-            x[st] = 0.0;
-#pragma unroll
-            for (int w = 0; w < kMaxWords; w++) cw[st][w] = 0;
-            if (s < s1) {
-                const cplx<double> cf = coef[s];
-                if (is_g) {
-                    const cplx<T> gv = g[s * net.Mpad + j];
-                    const double gr = double(gv.re), gi = conj_g ? -double(gv.im) : double(gv.im);
-                    if (conj_g == 2)   // coef_s |g_sj|^2 (diagonal of S)
-                        x[st] = imag_part ? 0.0 : cf.re * (gr * gr + gi * gi);
-                    else
-                        x[st] = imag_part ? cf.re * gi + cf.im * gr : cf.re * gr - cf.im * gi;
-                } else if (is_coef) {
-                    x[st] = imag_part ? cf.im : cf.re;
-                }
-#pragma unroll
-                for (int w = 0; w < kMaxWords; w++) cw[st][w] = w < words ? confs[s * words + w] : 0;
-            }
-        }
-#pragma unroll
-        for (int st = 0; st < kStage; st++) {
-#pragma unroll
-            for (int t = 0; t < kRowTilesPerWave; t++) {
-                if (vt0 + t < vtiles) {
-                    const int v = (vt0 + t) * 16 + (lane & 15);
-                    double a = 0.0;
-                    if (v < net.N) {
-                        const uint64_t word = v < 64 ? cw[st][0] : v < 128 ? cw[st][1] : v < 192 ? cw[st][2] : cw[st][3];
-                        a = ((word >> (v & 63)) & 1) ? 1.0 : -1.0;
-                    } else if (v == net.N) {
-                        a = 1.0;
-                    }
-                    acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, x[st], acc[t], 0, 0, 0);
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < kRowTilesPerWave; t++) {
-        if (vt0 + t < vtiles) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                // f64 16x16x4 result layout: item r of lane l is row l/16 + 4 r, column l%16
-                const int v = (vt0 + t) * 16 + (lane >> 4) + 4 * r;
-                partial[(int64_t(blockIdx.y) * vpad + v) * ncols + col] = acc[t][r];
-            }
-        }
-    }
-}
-
-__global__ void sum_partials_kernel(const double* partial, int chunks, int64_t n, double* out) {
-    const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    double acc = 0.0;
-    for (int c = 0; c < chunks; c++) acc += partial[c * n + e];
-    out[e] = acc;
-}
-
-// Yw[v][j], Yb[j], Ya[v] from the GEMM result Y[vpad][ncols]
-__global__ void split_spin_gemm_kernel(const double* Y, int N, int Mpad, int ncols, cplx<double>* Yw,
-                                       cplx<double>* Yb, cplx<double>* Ya) {
-    const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const int64_t nw = int64_t(N + 1) * Mpad;
-    if (e < nw) {
-        const int v = int(e / Mpad), j = int(e % Mpad);
-        const cplx<double> y = {Y[int64_t(v) * ncols + 2 * j], Y[int64_t(v) * ncols + 2 * j + 1]};
-        if (v < N) {
-            if (Yw) Yw[e] = y;
-        } else if (Yb) {
-            Yb[j] = y;
-        }
-    } else if (e < nw + N && Ya) {
-        const int v = int(e - nw);
-        Ya[v] = {Y[int64_t(v) * ncols + 2 * Mpad], Y[int64_t(v) * ncols + 2 * Mpad + 1]};
-    }
-}
-
-// u_s = sum_i s_i va_i + sum_j g_sj (vb_j + SV_sj)
-template <typename T, int U>
-__global__ __launch_bounds__(kBlock) void structured_Ov_kernel(DenseView<T> net, const uint64_t* confs,
-                                                               int words, const cplx<T>* g,
-                                                               const cplx<T>* SV, const cplx<double>* vb,
-                                                               const cplx<double>* va, int64_t count,
-                                                               cplx<double>* u_out) {
-    const int lane = threadIdx.x & 63;
-    const int64_t s = int64_t(blockIdx.x) * kWavesPerBlock + uniform_int(threadIdx.x >> 6);
-    if (s >= count) return;
-    const Conf c = load_conf(confs, s, words);
-    double re = 0, im = 0;
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-        const int j = lane + 64 * u;
-        if (j < net.M) {
-            const cplx<T> gv = g[s * net.Mpad + j];
-            const cplx<T> sv = SV[s * net.Mpad + j];
-            double xr = double(sv.re), xi = double(sv.im);
-            if (vb) {
-                xr += vb[j].re;
-                xi += vb[j].im;
-            }
-            re += double(gv.re) * xr - double(gv.im) * xi;
-            im += double(gv.re) * xi + double(gv.im) * xr;
-        }
-    }
-    if (va) {
-        for (int i = lane; i < net.N; i += 64) {
-            const double si = spin_bit(c, i) ? 1.0 : -1.0;
-            re += si * va[i].re;
-            im += si * va[i].im;
-        }
-    }
-    re = wave_sum(re);
-    im = wave_sum(im);
-    if (lane == 0) u_out[s] = {re, im};
-}
-
 // bf16 of x rounded to nearest even (the host's to_bf16 bit for bit)
 __device__ inline uint16_t bf16_rne(float x) {
     const uint32_t b = __float_as_uint(x);
@@ -702,14 +529,6 @@ void launch_enumerate_confs(uint64_t* confs, int64_t first_index, int64_t count,
 void launch_enumerate_paulis(uint64_t* confs, int64_t first_index, int64_t count, hipStream_t stream) {
     if (count <= 0) return;
     enumerate_paulis_kernel<<<unsigned((count + 255) / 256), 256, 0, stream>>>(confs, first_index, count);
-    ANN_LAUNCH_CHECK();
-}
-
-template <typename T>
-void launch_theta_valu(const DenseView<T>& net, const uint64_t* confs, int words, int64_t count,
-                       cplx<T>* theta, hipStream_t stream) {
-    if (count <= 0) return;
-    theta_valu_kernel<T><<<unsigned(count), kBlock, 0, stream>>>(net, confs, words, count, theta);
     ANN_LAUNCH_CHECK();
 }
 
@@ -854,52 +673,7 @@ void launch_materialize_ok(const DenseView<T>& net, const uint64_t* confs, int w
     ANN_LAUNCH_CHECK();
 }
 
-template <typename T>
-void launch_spin_weighted_sums(const DenseView<T>& net, const uint64_t* confs, int words, const cplx<T>* g,
-                               int conj_g, const cplx<double>* coef, int64_t count, cplx<double>* Yw,
-                               cplx<double>* Yb, cplx<double>* Ya, hipStream_t stream) {
-    if (count <= 0) return;
-    const int vpad = (net.N + 1 + 15) / 16 * 16;
-    const int ncols = 2 * net.Mpad + 16;
-    const int ctiles = ncols / 16;
-    const int zgroups = (vpad / 16 + kRowTilesPerWave - 1) / kRowTilesPerWave;
-    int64_t chunks = std::max<int64_t>(1, 4096 / (int64_t(ctiles) * zgroups));
-    chunks = std::min<int64_t>(chunks, (count + 63) / 64);
-    int64_t chunk = (count + chunks - 1) / chunks;
-    chunk = (chunk + 3) / 4 * 4;
-    chunks = (count + chunk - 1) / chunk;
-    const int64_t n = int64_t(vpad) * ncols;
-    double* partial = nullptr;
-    ANN_HIP_CHECK(hipMallocAsync(reinterpret_cast<void**>(&partial), sizeof(double) * n * (chunks + 1), stream));
-    double* full = partial + n * chunks;
-    const dim3 grid{unsigned(ctiles), unsigned(chunks), unsigned(zgroups)};
-    spin_gemm_kernel<T><<<grid, 64, 0, stream>>>(net, confs, words, g, conj_g, coef, count, chunk, vpad, ncols,
-                                                 partial);
-    ANN_LAUNCH_CHECK();
-    sum_partials_kernel<<<unsigned((n + 255) / 256), 256, 0, stream>>>(partial, int(chunks), n, full);
-    ANN_LAUNCH_CHECK();
-    const int64_t ns = int64_t(net.N + 1) * net.Mpad + net.N;
-    split_spin_gemm_kernel<<<unsigned((ns + 255) / 256), 256, 0, stream>>>(full, net.N, net.Mpad, ncols, Yw, Yb, Ya);
-    ANN_LAUNCH_CHECK();
-    ANN_HIP_CHECK(hipFreeAsync(partial, stream));
-}
-
-template <typename T>
-void launch_structured_Ov(const DenseView<T>& net, const uint64_t* confs, int words, const cplx<T>* g,
-                          const cplx<T>* SV, const cplx<double>* vb, const cplx<double>* va, int64_t count,
-                          cplx<double>* u, hipStream_t stream) {
-    if (count <= 0) return;
-    dispatch_u(net.Mpad / 64, [&](auto tag) {
-        constexpr int U = std::decay_t<decltype(tag)>::value;
-        structured_Ov_kernel<T, U><<<grid_waves(count), kBlock, 0, stream>>>(net, confs, words, g, SV, vb, va,
-                                                                              count, u);
-    });
-    ANN_LAUNCH_CHECK();
-}
-
 #define ANN_INSTANTIATE(T)                                                                                   \
-    template void launch_theta_valu<T>(const DenseView<T>&, const uint64_t*, int, int64_t, cplx<T>*,        \
-                                       hipStream_t);                                                         \
     template void launch_net_log_psi<T>(const DenseView<T>&, const cplx<T>*, int64_t, cplx<double>,        \
                                         cplx<double>*, double*, hipStream_t);                                \
     template void launch_mc_sweep<T>(const DenseView<T>&, uint64_t*, cplx<T>*, int, int, int, int64_t,      \
@@ -908,13 +682,7 @@ void launch_structured_Ov(const DenseView<T>& net, const uint64_t* confs, int wo
                                          int64_t, cplx<double>*, hipStream_t);                               \
     template void launch_g_factor<T>(const DenseView<T>&, const cplx<T>*, int64_t, cplx<T>*, hipStream_t);  \
     template void launch_materialize_ok<T>(const DenseView<T>&, const uint64_t*, int, const cplx<T>*,       \
-                                           int64_t, const cplx<double>*, cplx<T>*, hipStream_t);             \
-    template void launch_spin_weighted_sums<T>(const DenseView<T>&, const uint64_t*, int, const cplx<T>*,   \
-                                               int, const cplx<double>*, int64_t, cplx<double>*,             \
-                                               cplx<double>*, cplx<double>*, hipStream_t);                   \
-    template void launch_structured_Ov<T>(const DenseView<T>&, const uint64_t*, int, const cplx<T>*,        \
-                                          const cplx<T>*, const cplx<double>*, const cplx<double>*, int64_t, \
-                                          cplx<double>*, hipStream_t);
+                                           int64_t, const cplx<double>*, cplx<T>*, hipStream_t);
 
 ANN_INSTANTIATE(float)
 ANN_INSTANTIATE(double)

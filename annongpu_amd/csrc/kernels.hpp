@@ -93,9 +93,9 @@ void launch_enumerate_confs(uint64_t* confs, int64_t first_index, int64_t count,
 // bit 2i of the index as its a bit and bit 2i + 1 as its b bit; confs [count][2]
 void launch_enumerate_paulis(uint64_t* confs, int64_t first_index, int64_t count, hipStream_t stream);
 
-template <typename T>
-void launch_theta_valu(const DenseView<T>& net, const uint64_t* confs, int words, int64_t count,
-                       cplx<T>* theta, hipStream_t stream);
+// fp64: theta = S Wd + b, a sum over the sites in ascending order from b (sr_dense64.hip)
+void launch_theta64(const DenseView<double>& net, const uint64_t* confs, int words, int64_t count,
+                    cplx<double>* theta, hipStream_t stream);
 
 // theta = S * Wd + b on MFMA: spins are exact in bf16, Wd is split into three bf16
 // terms (hi, mid, lo) and accumulated in fp32.  wfrag is the fragment-ordered
@@ -142,25 +142,22 @@ void launch_materialize_ok(const DenseView<T>& net, const uint64_t* confs, int w
                            const cplx<T>* g, int64_t count, const cplx<double>* center,
                            cplx<T>* O, hipStream_t stream);
 
-// Yw[v][j] = sum_s coef_s spin_sv X_sj, Yb[j] = sum_s coef_s X_sj,
-// Ya[v] = sum_s coef_s spin_sv, fp64 accumulation (fp64 MFMA).
-// X_sj = g_sj (conj_g = 0), conj(g_sj) (1) or |g_sj|^2 (2).
-template <typename T>
-void launch_spin_weighted_sums(const DenseView<T>& net, const uint64_t* confs, int words,
-                               const cplx<T>* g, int conj_g, const cplx<double>* coef,
-                               int64_t count, cplx<double>* Yw, cplx<double>* Yb,
-                               cplx<double>* Ya, hipStream_t stream);
-
-// u_s = coef_s * (O_s . v - shift_u) for the structured O of a dense net; V is the
-// reindexed W part of v ([N][Mpad]), vb the bias part, va the visible part.
-template <typename T>
-void launch_structured_Ov(const DenseView<T>& net, const uint64_t* confs, int words,
-                          const cplx<T>* g, const cplx<T>* SV, const cplx<double>* vb,
-                          const cplx<double>* va, int64_t count, cplx<double>* u,
-                          hipStream_t stream);
+// y = sum_s coef_s O_s (conj_g = 0) or sum_s coef_s conj(O_s) (1) in parameter order, + shift
+// v, fp64 (fp64 MFMA; sr_dense64.hip).  work: spin_sums64_work doubles; ypart (optional):
+// Re(v^H y) of every 64 parameters, spin_sums64_parts of them filled up to a multiple of 4
+size_t spin_sums64_work(int N, int Mpad, int64_t count);
+int spin_sums64_parts(int64_t num_params);
+void launch_spin_sums64(const DenseView<double>& net, const uint64_t* confs, int words, const cplx<double>* g,
+                        int conj_g, const cplx<double>* coef, int64_t count, double* work, double shift,
+                        const cplx<double>* v, cplx<double>* y, double* ypart, hipStream_t stream);
+// Yb[j] = sum_s coef_s X_sj with X = g (mode 0), conj g (1) or |g|^2 (2)
+void launch_spin_bias64(const DenseView<double>& net, const uint64_t* confs, int words, const cplx<double>* g,
+                        int mode, const cplx<double>* coef, int64_t count, double* work, cplx<double>* Yb,
+                        hipStream_t stream);
 
 // weighted fp64 reductions
-// the spin GEMM of launch_spin_weighted_sums on bf16 matrix cores (fp32 accumulation
+// Yw[v][j] = sum_s coef_s spin_sv X_sj, Yb[j] = sum_s coef_s X_sj, Ya[v] = sum_s coef_s
+// spin_sv with X_sj = g_sj (mode 0), conj(g_sj) (1) or |g_sj|^2 (2) on bf16 matrix cores (fp32 accumulation
 // per sample chunk, chunks added in fp64)
 // ws (optional): the caller's transposed spin bits of the samples (launch_spin_bits with
 // the plan's vpad) and workspace of spin_sums_work sizes; without it the call builds the
@@ -228,6 +225,15 @@ struct CgDir {
     const int* done = nullptr;
     cplx<double>* p_new = nullptr;
 };
+// fp64 (sr_dense64.hip): re-indexed v (V [N][Mpad], vb, va) and the partials of <O>.v
+// (dpart, [sr_dot_parts64()][2]), then u_s = w_s (O_s.v - <O>.v)
+int sr_dot_parts64();
+void launch_sr_prepare64(const DenseView<double>& net, const int* inv, const cplx<double>* v, const CgDir& dir,
+                         const cplx<double>* obar, double* dpart, cplx<double>* va, cplx<double>* vb,
+                         cplx<double>* V, hipStream_t stream);
+void launch_sr_ov64(const DenseView<double>& net, const uint64_t* confs, int words, const cplx<double>* g,
+                    const cplx<double>* V, const cplx<double>* vb, const cplx<double>* va, const double* w,
+                    const double* dpart, int64_t count, cplx<double>* u, hipStream_t stream);
 int sr_y_parts(const DenseView<float>& net, const WParamMap& wm);
 int sr_kt32(int N);
 int sr_ov_pairs(int M);

@@ -9,11 +9,6 @@ namespace ann {
 void launch_init_chains(uint64_t* confs, int num_chains, int words, int N, int move, int total_z,
                         uint32_t call_index, uint64_t seed, hipStream_t stream);
 
-// inv[vis][j] ([N][Mpad]): the unique i with conn(i, j) = vis, -1 if none, -2 if several
-template <typename T>
-void launch_unpack_v(const DenseView<T>& net, const int* inv, const cplx<double>* v, cplx<double>* va,
-                     cplx<double>* vb, cplx<T>* V, hipStream_t stream);
-
 void launch_pack_y(int layout, int N, int M, int Mpad, int C, const uint32_t* conn, const cplx<double>* Ya,
                    const cplx<double>* Yb, const cplx<double>* Yw, const cplx<double>* v, double shift, int P,
                    cplx<double>* y, hipStream_t stream);
@@ -33,6 +28,11 @@ void launch_cg_dir_dev(cplx<double>* p, const cplx<double>* z, const double* rz_
 // preconditioned CG (cg.hip): dot products as kCgParts block partials [b][4] = (r^H z, -, r^H r, -);
 // a matvec's partials of p^H Ap are [b][2]
 constexpr int kCgParts = 256;
+// partials of a real dot product: n <= 256 of them, element 0 of [n][2] or the sums of [n][4]
+struct DotParts {
+    const double* p = nullptr;
+    int n = 0, stride = 2;
+};
 void launch_pcg_init(const cplx<double>* r, cplx<double>* z, cplx<double>* p, const double* diag, double shift,
                      int64_t n, int64_t jac_end, double* part, hipStream_t stream);
 
@@ -104,7 +104,7 @@ void launch_pcg_pap(const cplx<double>* p, const cplx<double>* Ap, int64_t n, do
 // r^H z is the sum of slots 0 (Jacobi) and 1 (K-FAC) of the partials.
 void launch_pcg_step(cplx<double>* x, cplx<double>* r, cplx<double>* z, const cplx<double>* p,
                      const cplx<double>* Ap, const double* diag, double shift, int64_t n, int64_t jac_end,
-                     const double* rzpart, const double* apart, int a_parts, double* newpart, const int* done,
+                     const double* rzpart, const DotParts& apart, double* newpart, const int* done,
                      hipStream_t stream);
 void launch_pcg_dir(cplx<double>* p, const cplx<double>* z, int64_t n, const double* newpart, const double* oldpart,
                     const int* done, hipStream_t stream);

@@ -836,7 +836,7 @@ const DevicePauliOp& Operator::device_pauli() {
 void compute_theta(Psi& psi, const uint64_t* confs, int64_t count, Samples& out, int64_t offset) {
     ScopedTimer timer("theta");
     if (psi.precision == 0) {
-        launch_theta_valu<double>(psi.view64(), confs, psi.words, count, out.th64.p + offset * psi.Mpad, S());
+        launch_theta64(psi.view64(), confs, psi.words, count, out.th64.p + offset * psi.Mpad, S());
     } else {
         auto v = psi.view32();
         launch_theta_mfma(v, psi.wfrag.p, psi.npad, confs, psi.words, count, out.th32.p + offset * psi.Mpad, S());
@@ -1201,16 +1201,18 @@ void g_factor_padded(const DenseView<T>& net, const cplx<T>* theta, int64_t coun
         ANN_HIP_CHECK(hipMemsetAsync(g.p + size_t(count) * net.Mpad, 0, sizeof(cplx<T>) * (pad - count) * net.Mpad, S()));
 }
 
-// weighted sums of the structured O, packed in parameter order: out = sum_s coef_s O_s (or conj O_s)
+// weighted sums of the structured O, packed in parameter order: out = sum_s coef_s O_s (or
+// conj O_s) + shift v; without out, sum_s coef_s |g_sj|^2 into t.Yb.  fp64 with ypart:
+// the partials of Re(v^H out)
 template <typename T>
 void structured_sums(Tdvp& t, const DenseView<T>& net, const uint64_t* confs, int words, const cplx<T>* g,
                      int conj_g, const cplx<double>* coef, int64_t count, cplx<double>* out, double shift,
-                     const cplx<double>* v) {
-    t.Yw.ensure(size_t(net.N) * net.Mpad);
+                     const cplx<double>* v, double* ypart = nullptr) {
     t.Yb.ensure(net.Mpad);
-    t.Ya.ensure(net.N);
     ScopedTimer timer("spin_sums");
     if constexpr (sizeof(T) == 4) {
+        t.Yw.ensure(size_t(net.N) * net.Mpad);
+        t.Ya.ensure(net.N);
         // the transposed spin bits of this evaluation's samples are built once and
         // shared with the S.v products and the K-FAC set-up; the workspace persists
         const SpinPlan plan = spin_plan(net.N, net.M, net.Mpad, count, true);
@@ -1224,11 +1226,16 @@ void structured_sums(Tdvp& t, const DenseView<T>& net, const uint64_t* confs, in
         t.ss_c32.ensure(size_t(sr_count_pad(count)));
         const SpinSumsWork ws{t.spin_bits.p, t.ss_partial.p, t.ss_full.p, t.ss_c32.p};
         launch_spin_sums_bf16(net, confs, words, g, conj_g, coef, count, t.Yw.p, t.Yb.p, t.Ya.p, S(), &ws);
-    } else
-        launch_spin_weighted_sums<T>(net, confs, words, g, conj_g, coef, count, t.Yw.p, t.Yb.p, t.Ya.p, S());
-    if (out)
-        launch_pack_y(net.layout, net.N, net.M, net.Mpad, net.C, net.conn, t.Ya.p, t.Yb.p, t.Yw.p, v, shift,
-                      net.num_params, out, S());
+        if (out)
+            launch_pack_y(net.layout, net.N, net.M, net.Mpad, net.C, net.conn, t.Ya.p, t.Yb.p, t.Yw.p, v, shift,
+                          net.num_params, out, S());
+    } else {
+        t.ss_work64.ensure(spin_sums64_work(net.N, net.Mpad, count));
+        if (out)
+            launch_spin_sums64(net, confs, words, g, conj_g, coef, count, t.ss_work64.p, shift, v, out, ypart, S());
+        else
+            launch_spin_bias64(net, confs, words, g, conj_g, coef, count, t.ss_work64.p, t.Yb.p, S());
+    }
 }
 
 // K-FAC factor buffers of the Tdvp's current sizes
@@ -1528,26 +1535,14 @@ void tdvp_S_dot_generic(Tdvp& t, const cplx<double>* v, double shift, cplx<doubl
     launch_ok_colsum<T>(O.p, t.count, P, t.u.p, 1, shift, v, t.part.p, y, S());
 }
 
+// y = (S + shift) v for the structured O of a dense net, on bf16 matrix cores in the fp32
+// mode and on fp64 ones in the fp64 mode.  With dir, v is the CG direction that the first
+// kernel forms (dir.p_new).  vy: the partials of v^H y; left empty in the fp64 mode for
+// more than 256 kCgParts parameters, where a thread of the kernel that adds them sums
+// several parameters first.
 template <typename T>
-struct Ws;
-template <>
-struct Ws<float> {
-    static DevBuf<cplx<float>>& V(Tdvp& t) { return t.V32; }
-    static DevBuf<cplx<float>>& SV(Tdvp& t) { return t.SV32; }
-    static DevBuf<cplx<float>>& zero(Tdvp& t) { return t.zero32; }
-};
-template <>
-struct Ws<double> {
-    static DevBuf<cplx<double>>& V(Tdvp& t) { return t.V64; }
-    static DevBuf<cplx<double>>& SV(Tdvp& t) { return t.SV64; }
-    static DevBuf<cplx<double>>& zero(Tdvp& t) { return t.zero64; }
-};
-
-// y = (S + shift) v for the structured O of a dense net.  The fp32 path runs the
-// fused bf16 matrix-core pipeline and also leaves the partials of v^H y (*ypart).
-template <typename T>
-void tdvp_S_dot_t(Tdvp& t, const cplx<double>* v, double shift, cplx<double>* y, const double** ypart,
-                  int* yparts, const CgDir* dir = nullptr) {
+void tdvp_S_dot_t(Tdvp& t, const cplx<double>* v, double shift, cplx<double>* y, DotParts* vy,
+                  const CgDir* dir = nullptr) {
     const int P = int(t.P);
     DenseView<T> net{};
     net.N = t.N;
@@ -1603,38 +1598,25 @@ void tdvp_S_dot_t(Tdvp& t, const cplx<double>* v, double shift, cplx<double>* y,
             ScopedTimer timer("sr_y", timed);
             launch_sr_y_bf16(net, wm, v, shift, plan, ws, y, S());
         }
-        if (ypart) *ypart = t.ypart.p;
-        if (yparts) *yparts = sr_y_parts(net, wm);
+        if (vy) *vy = {t.ypart.p, sr_y_parts(net, wm), 2};
         return;
     } else {
-        auto& V = Ws<T>::V(t);
-        auto& SV = Ws<T>::SV(t);
-        auto& zero = Ws<T>::zero(t);
-        t.c1.ensure(2);
-        t.dot_scratch.ensure(256);
-        V.ensure(size_t(t.N) * t.Mpad);
-        SV.ensure(size_t(t.count) * t.Mpad);
-        if (zero.n < size_t(t.Mpad)) {
-            zero.ensure(t.Mpad);
-            ANN_HIP_CHECK(hipMemsetAsync(zero.p, 0, sizeof(cplx<T>) * t.Mpad, S()));
-        }
+        t.dot_scratch.ensure(size_t(2) * sr_dot_parts64());
+        t.V64.ensure(size_t(t.N) * t.Mpad);
+        const bool deep = t.layout == LAYOUT_DEEP1;
         {
             ScopedTimer timer("sr_matvec");
-            launch_unpack_v<T>(net, t.inv.p, v, t.va.p, t.vb.p, V.p, S());
-            DenseView<T> vnet = net;
-            vnet.Wd = V.p;
-            vnet.b = zero.p;
-            const cplx<double>* vb = t.layout == LAYOUT_DEEP1 ? t.vb.p : nullptr;
-            const cplx<double>* va = t.layout == LAYOUT_DEEP1 ? t.va.p : nullptr;
-            launch_theta_valu<T>(vnet, t.confs.p, t.words, t.count, SV.p, S());
-            launch_structured_Ov<T>(net, t.confs.p, t.words, g.p, SV.p, vb, va, t.count, t.u.p, S());
-            launch_dot2(t.Obar.p, v, nullptr, nullptr, P, 0, t.dot_scratch.p, reinterpret_cast<double*>(t.c1.p),
-                        S());
-            launch_center_scale(t.u.p, t.w.p, reinterpret_cast<const double*>(t.c1.p), t.count, S());
+            launch_sr_prepare64(net, t.inv.p, v, dir ? *dir : CgDir{}, t.Obar.p, t.dot_scratch.p, t.va.p, t.vb.p,
+                                t.V64.p, S());
+            launch_sr_ov64(net, t.confs.p, t.words, g.p, t.V64.p, deep ? t.vb.p : nullptr, deep ? t.va.p : nullptr,
+                           t.w.p, t.dot_scratch.p, t.count, t.u.p, S());
         }
-        structured_sums<T>(t, net, t.confs.p, t.words, g.p, 1, t.u.p, t.count, y, shift, v);
-        if (ypart) *ypart = nullptr;
-        if (yparts) *yparts = 0;
+        const int parts = (spin_sums64_parts(P) + 3) / 4;
+        const bool fused = vy && parts <= kCgParts;
+        if (fused) t.ypart.ensure(size_t(parts) * 4);
+        structured_sums<T>(t, net, t.confs.p, t.words, g.p, 1, t.u.p, t.count, y, shift, v,
+                           fused ? t.ypart.p : nullptr);
+        if (fused) *vy = {t.ypart.p, parts, 4};
     }
 }
 
@@ -1665,17 +1647,22 @@ void ok_weighted_sum_t(Psi& psi, Samples& s, const cplx<double>* coef, int conj,
     DenseView<T> net = Prec<T>::view(psi);
     DevBuf<cplx<T>> g;
     g_factor_padded<T>(net, Prec<T>::th(s).p, s.count, g);
-    DevBuf<cplx<double>> Yw, Yb, Ya;
-    Yw.ensure(size_t(psi.N) * psi.Mpad);
-    Yb.ensure(psi.Mpad);
-    Ya.ensure(psi.N);
-    if constexpr (sizeof(T) == 4)
+    if constexpr (sizeof(T) == 4) {
+        DevBuf<cplx<double>> Yw, Yb, Ya;
+        Yw.ensure(size_t(psi.N) * psi.Mpad);
+        Yb.ensure(psi.Mpad);
+        Ya.ensure(psi.N);
         launch_spin_sums_bf16(net, s.confs.p, s.words, g.p, conj, coef, s.count, Yw.p, Yb.p, Ya.p, S());
-    else
-        launch_spin_weighted_sums<T>(net, s.confs.p, s.words, g.p, conj, coef, s.count, Yw.p, Yb.p, Ya.p, S());
-    launch_pack_y(net.layout, net.N, net.M, net.Mpad, net.C, net.conn, Ya.p, Yb.p, Yw.p, nullptr, 0.0,
-                  psi.num_params, out, S());
-    Runtime::get().sync();
+        launch_pack_y(net.layout, net.N, net.M, net.Mpad, net.C, net.conn, Ya.p, Yb.p, Yw.p, nullptr, 0.0,
+                      psi.num_params, out, S());
+        Runtime::get().sync();   // before the buffers go
+    } else {
+        DevBuf<double> work;
+        work.ensure(spin_sums64_work(psi.N, psi.Mpad, s.count));
+        launch_spin_sums64(net, s.confs.p, s.words, g.p, conj, coef, s.count, work.p, 0.0, nullptr, out, nullptr,
+                           S());
+        Runtime::get().sync();
+    }
 }
 
 }  // namespace
@@ -1948,9 +1935,8 @@ void tdvp_O_samples(Tdvp& t, cd* out) {
         o_samples_t<float>(t, out);
 }
 
-void tdvp_S_dot(Tdvp& t, const cplx<double>* v, double shift, cplx<double>* y, const double** ypart, int* yparts) {
-    if (ypart) *ypart = nullptr;
-    if (yparts) *yparts = 0;
+void tdvp_S_dot(Tdvp& t, const cplx<double>* v, double shift, cplx<double>* y, DotParts* vy) {
+    if (vy) *vy = {};
     if (!t.has_samples) throw std::logic_error("TDVP.eval must run before S_dot_vector");
     if (t.generic) {
         if (t.precision == 0)
@@ -1960,22 +1946,25 @@ void tdvp_S_dot(Tdvp& t, const cplx<double>* v, double shift, cplx<double>* y, c
         return;
     }
     if (t.precision == 0)
-        tdvp_S_dot_t<double>(t, v, shift, y, ypart, yparts);
+        tdvp_S_dot_t<double>(t, v, shift, y, vy);
     else
-        tdvp_S_dot_t<float>(t, v, shift, y, ypart, yparts);
+        tdvp_S_dot_t<float>(t, v, shift, y, vy);
 }
 
-const cplx<double>* tdvp_S_dot_dir(Tdvp& t, const CgDir& dir, double shift, cplx<double>* y, const double** ypart,
-                                   int* yparts) {
+const cplx<double>* tdvp_S_dot_dir(Tdvp& t, const CgDir& dir, double shift, cplx<double>* y, DotParts* vy) {
+    if (vy) *vy = {};
     if (!t.has_samples) throw std::logic_error("TDVP.eval must run before S_dot_vector");
-    if (!t.generic && t.precision != 0) {
-        // the fp32 structured matvec forms the direction inside its first kernel
-        tdvp_S_dot_t<float>(t, dir.p_new, shift, y, ypart, yparts, &dir);
+    if (!t.generic) {
+        // the structured matvecs form the direction inside their first kernel
+        if (t.precision == 0)
+            tdvp_S_dot_t<double>(t, dir.p_new, shift, y, vy, &dir);
+        else
+            tdvp_S_dot_t<float>(t, dir.p_new, shift, y, vy, &dir);
         return dir.p_new;
     }
     cplx<double>* p = const_cast<cplx<double>*>(dir.p_old);
     launch_pcg_dir(p, dir.z, int64_t(t.P), dir.newpart, dir.oldpart, dir.done, S());
-    tdvp_S_dot(t, p, shift, y, ypart, yparts);
+    tdvp_S_dot(t, p, shift, y, vy);
     return p;
 }
 
@@ -2164,10 +2153,11 @@ int tdvp_solve(Tdvp& t, double shift, int method, double rtol, int max_iter, cd*
     while (!stop && it < max_iter) {
         const double* cur = part.p + size_t(it) * stride;
         double* nxt = part.p + size_t(it + 1) * stride;
-        const double* ypart = nullptr;
-        int yparts = 0;
+        // (the K-FAC step reads partials of stride 2 only)
+        DotParts vy;
+        DotParts* const want = kfac && t.precision == 0 ? nullptr : &vy;
         if (it == 0) {
-            tdvp_S_dot(t, pk, shift, Ap.p, &ypart, &yparts);
+            tdvp_S_dot(t, pk, shift, Ap.p, want);
         } else {
             CgDir dir;
             dir.z = z.p;
@@ -2177,16 +2167,15 @@ int tdvp_solve(Tdvp& t, double shift, int method, double rtol, int max_iter, cd*
             dir.parts = kCgParts;
             dir.done = done.p;
             dir.p_new = spare;
-            const cplx<double>* pn = tdvp_S_dot_dir(t, dir, shift, Ap.p, &ypart, &yparts);
+            const cplx<double>* pn = tdvp_S_dot_dir(t, dir, shift, Ap.p, want);
             if (pn == spare) {
                 spare = const_cast<cplx<double>*>(pk);
                 pk = pn;
             }
         }
-        if (!ypart) {
+        if (!vy.p) {
             launch_pcg_pap(pk, Ap.p, P, apart.p, S());
-            ypart = apart.p;
-            yparts = kCgParts;
+            vy = {apart.p, kCgParts, 2};
         }
         if (kfac) {
             ScopedTimer timer("kfac_step", (it & 15) == 0);
@@ -2201,14 +2190,14 @@ int tdvp_solve(Tdvp& t, double shift, int method, double rtol, int max_iter, cd*
             a.shift = shift;
             a.jac_end = jac_end;
             a.rzpart = cur;
-            a.apart = ypart;
-            a.a_parts = yparts;
+            a.apart = vy.p;
+            a.a_parts = vy.n;
             a.newpart = nxt;
             a.done = done.p;
             launch_kfac_step(kv, a, S());
             r_cur = a.r_out;
         } else {
-            launch_pcg_step(x.p, r.p, z.p, pk, Ap.p, diag, shift, P, jac_end, cur, ypart, yparts, nxt, done.p, S());
+            launch_pcg_step(x.p, r.p, z.p, pk, Ap.p, diag, shift, P, jac_end, cur, vy, nxt, done.p, S());
         }
         it++;
         if (it % check == 0 || it == max_iter) {

@@ -420,8 +420,8 @@ struct Tdvp {
     DevBuf<double> diag;   // diagonal of S (Jacobi preconditioner)
     // S.v workspace (grow-only)
     DevBuf<cplx<double>> va, vb, u, c1, Yw, Yb, Ya;
-    DevBuf<cplx<float>> V32, SV32, zero32;
-    DevBuf<cplx<double>> V64, SV64, zero64;
+    DevBuf<cplx<double>> V64;
+    DevBuf<double> ss_work64;
     DevBuf<uint16_t> frag;       // bf16x3 fragments of v (fp32 mode)
     DevBuf<cplx<float>> upart;   // per column pair partial O.v (fp32 mode)
     DevBuf<cplx<float>> u32;     // w (O.v - <O>.v) per sample (fp32 mode)
@@ -501,10 +501,11 @@ cd expectation_exp_fast(Operator& op, Psi& psi, Ensemble& ens);
 // <op> in psi from the samples of psi_sampling weighted by |psi / psi_sampling|^2
 cd expectation_reweighted(Operator& op, Psi& psi, Psi& psi_sampling, Ensemble& ens);
 void tdvp_eval(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with_S);
-// y = (S + shift) v on the device; when the matvec also produced the block partials
-// of v^H y, *ypart / *yparts describe them ([yparts][2]), else they are null / 0
+// y = (S + shift) v on the device; *vy: the partials of v^H y when the matvec also produced
+// them, else empty
+struct DotParts;
 void tdvp_S_dot(Tdvp& t, const cplx<double>* v_dev, double shift, cplx<double>* y_dev,
-                const double** ypart = nullptr, int* yparts = nullptr);
+                DotParts* vy = nullptr);
 // method 0 Cholesky, 1 Jacobi-preconditioned CG, 3 K-FAC-preconditioned CG (dense
 // nets), the CG methods from x0 (zero when x0 is null)
 int tdvp_solve(Tdvp& t, double shift, int method, double rtol, int max_iter, cd* x, int* iters, double* res,

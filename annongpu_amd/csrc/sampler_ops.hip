@@ -44,52 +44,6 @@ __global__ void init_chains_kernel(uint64_t* confs, int num_chains, int words, i
     for (int k = 0; k < words; k++) confs[int64_t(c) * words + k] = w[k];
 }
 
-// v (reference parameter order) -> va [N], vb [Mpad], V [N][Mpad] (W part re-indexed
-// onto visible units: V[conn(i,j)][j] += v_W(i,j)); one thread per V element
-template <typename T>
-__global__ void unpack_v_kernel(DenseView<T> net, const int* inv, const cplx<double>* v, cplx<double>* va,
-                                cplx<double>* vb, cplx<T>* V) {
-    const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const int64_t nV = int64_t(net.N) * net.Mpad;
-    if (e < nV) {
-        const int vis = int(e / net.Mpad), j = int(e % net.Mpad);
-        double re = 0.0, im = 0.0;
-        if (j < net.M) {
-            if (net.layout == LAYOUT_RBM) {
-                const cplx<double> x = v[int64_t(vis) * net.M + j];
-                re = x.re;
-                im = x.im;
-            } else {
-                // inv[vis][j]: the unique i with conn(i, j) = vis, -1 if none, -2 if several
-                const int i0 = inv[e];
-                if (i0 >= 0) {
-                    const cplx<double> x = v[net.N + net.M + int64_t(i0) * net.M + j];
-                    re = x.re;
-                    im = x.im;
-                } else if (i0 == -2) {
-                    for (int i = 0; i < net.C; i++) {
-                        if (int(net.conn[int64_t(i) * net.M + j]) == vis) {
-                            const cplx<double> x = v[net.N + net.M + int64_t(i) * net.M + j];
-                            re += x.re;
-                            im += x.im;
-                        }
-                    }
-                }
-            }
-        }
-    V[e] = {T(re), T(im)};
-        return;
-    }
-    const int64_t e2 = e - nV;
-    if (e2 < net.Mpad) {
-        const int j = int(e2);
-        if (vb) vb[j] = (net.layout == LAYOUT_DEEP1 && j < net.M) ? v[net.N + j] : cplx<double>{0, 0};
-    } else if (e2 < int64_t(net.Mpad) + net.N) {
-        const int i = int(e2 - net.Mpad);
-        if (va) va[i] = net.layout == LAYOUT_DEEP1 ? v[i] : cplx<double>{0, 0};
-    }
-}
-
 // y (reference order) from Ya, Yb, Yw (+ shift * v)
 __global__ void pack_y_kernel(int layout, int N, int M, int Mpad, int C, const uint32_t* conn,
                               const cplx<double>* Ya, const cplx<double>* Yb, const cplx<double>* Yw,
@@ -324,18 +278,6 @@ void launch_init_chains(uint64_t* confs, int num_chains, int words, int N, int m
                                                                       uint32_t(seed >> 32));
     ANN_LAUNCH_CHECK();
 }
-
-template <typename T>
-void launch_unpack_v(const DenseView<T>& net, const int* inv, const cplx<double>* v, cplx<double>* va,
-                     cplx<double>* vb, cplx<T>* V, hipStream_t stream) {
-    const int64_t n = int64_t(net.N) * net.Mpad + net.Mpad + net.N;
-    unpack_v_kernel<T><<<blocks_for(n), 256, 0, stream>>>(net, inv, v, va, vb, V);
-    ANN_LAUNCH_CHECK();
-}
-template void launch_unpack_v<float>(const DenseView<float>&, const int*, const cplx<double>*, cplx<double>*,
-                                     cplx<double>*, cplx<float>*, hipStream_t);
-template void launch_unpack_v<double>(const DenseView<double>&, const int*, const cplx<double>*, cplx<double>*,
-                                      cplx<double>*, cplx<double>*, hipStream_t);
 
 void launch_pack_y(int layout, int N, int M, int Mpad, int C, const uint32_t* conn, const cplx<double>* Ya,
                    const cplx<double>* Yb, const cplx<double>* Yw, const cplx<double>* v, double shift, int P,
