@@ -265,7 +265,18 @@ __global__ __launch_bounds__(kBlock) void mc_sweep_kernel(DenseView<T> net, uint
             // branch-free update of the angles (the decision is wave-uniform)
             const bool accept = d2 > T(0) || uu <= dexp(d2);
 #pragma unroll
-            for (int u = 0; u < U; u++) th[u] = accept ? z[u] : th[u];
+            for (int u = 0; u < U; u++) {
+                if constexpr (sizeof(T) == 8) {
+                    // by component: a choice between two structs of 16 bytes is compiled as one between
+                    // their addresses, which puts both arrays into scratch memory (45 sites, 90
+                    // units, 1,000 chains: 1.2 us a proposal with it, 0.5 without)
+                    const T zr = z[u].re, zi = z[u].im, tr = th[u].re, ti = th[u].im;
+                    th[u].re = accept ? zr : tr;
+                    th[u].im = accept ? zi : ti;
+                } else {
+                    th[u] = accept ? z[u] : th[u];
+                }
+            }
             cur = accept ? nxt : cur;
 #pragma unroll
             for (int k = 0; k < WORDS; k++) {
