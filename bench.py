@@ -379,7 +379,7 @@ def cnn_quench_leg(A, steps=2, warmup=1, progress=False, precision="fp32", shift
             "energy_max_rel_change": float(np.max(np.abs(E_steps - E_steps[0])) / abs(E_steps[0])),
             "failure": failure, "precision": precision, "shift": shift,
             "param_norm_per_step": pnorm,
-            "sweep_roofline": {"bound": "valu", "kernel": "cnn_mc_inc (local updates)",
+            "sweep_roofline": {"bound": "valu", "kernel": "cnn_pair_mc (second-layer updates)",
                                "achieved_tflops": work / (sweep_ms * 1e-3) / 1e12 if sweep_ms else None,
                                "peak_tflops": 157.3,
                                "frac": work / (sweep_ms * 1e-3) / 1e12 / 157.3 if sweep_ms else None}}
