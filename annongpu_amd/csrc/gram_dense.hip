@@ -5,7 +5,8 @@
 //   sum_s w O_k^* O_k' = sum_s (s_i s_i') (w conj(g_j) g_j'),
 // which depends on the unordered pairs {i, i'} (real, +-1) and {j, j'} (complex, Hermitian).
 // So S needs one real x complex product per pair of pairs, P^2 flop per sample, where
-// a complex Gram of the materialised O needs 4 P^2, and neither O nor its traffic.
+// a complex Gram of the materialised O needs 4 P^2, and neither O nor its traffic.  The sums are
+// of uncentred O: the caller takes this form only while no parameter's mean dominates its spread.
 //   pairs_gemm   T[site pair][unit pair] on v_mfma_f64_16x16x4_f64, signs from the
 //                transposed spin bits, the unit products formed into LDS once per 256 site pairs
 //   assemble     S[k][k'] = T - conj(m_k) m_k', m = <O>, read from the constant's row of T

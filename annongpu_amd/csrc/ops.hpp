@@ -123,6 +123,9 @@ void launch_precond(cplx<double>* z, const cplx<double>* r, const double* diag, 
                     hipStream_t stream);
 void launch_sr_diag(int layout, int N, int M, int Mpad, const double* wsum, const cplx<double>* Dj,
                     const cplx<double>* Obar, int P, double* diag, hipStream_t stream);
+// *out = number of parameters with |<O_k>|^2 > limit diag_k (or not a number)
+void launch_mean_dominated(const cplx<double>* Obar, const double* diag, int P, double limit, double* out,
+                           hipStream_t stream);
 void launch_rank1(cplx<double>* S, const cplx<double>* o, int P, double alpha, hipStream_t stream);
 template <typename Tin, typename Tout>
 void launch_convert(const cplx<Tin>* a, cplx<Tout>* b, int64_t n, hipStream_t stream);

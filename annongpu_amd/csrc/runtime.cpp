@@ -1310,7 +1310,7 @@ void tdvp_eval_t(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with_S) {
     t.Obar.ensure(P);
     t.Fd.ensure(P);
     t.diag.ensure(P);
-    t.sums.ensure(4);
+    t.sums.ensure(5);
     launch_weight_coef(s.w.p, nullptr, n, coef.p, S());
     const bool pre_kfac = t.kfac_hint && psi.N <= kKfacMaxSites && psi.M <= kKfacMaxUnits &&
                           (psi.layout == LAYOUT_RBM || t.inv_unique);
@@ -1363,16 +1363,30 @@ void tdvp_eval_t(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with_S) {
     ANN_HIP_CHECK(hipStreamWaitEvent(S(), t.join_ev.get(), 0));
     if (pre_kfac) ANN_HIP_CHECK(hipStreamWaitEvent(S(), t.join2_ev.get(), 0));
     launch_sr_diag(net.layout, net.N, net.M, net.Mpad, t.sums.p + 3, t.Yb.p, t.Obar.p, P, t.diag.p, S());
-    // F = sum w conj(O) E_loc - E conj(<O>) (TDVP.cu.template:300) = sum w (E_loc - E) conj(O)
-    launch_weight_coef_centered_dev(s.w.p, s.e_loc.p, t.sums.p, n, coef.p, S());
-    structured_sums<T>(t, net, s.confs.p, s.words, g.p, 1, coef.p, n, t.Fd.p, 0.0, nullptr);
+    // S from pairs of sites and pairs of units when nearly every (site, unit), the biases'
+    // constants included, carries a parameter: (N+1)^2 (M+1)^2 flop per sample against 4 P^2 for
+    // the Gram of the materialised O.  (They cross at a quarter of the pairs' count; the line is
+    // at a third, as the pairs' table has to be gathered.)
+    const double pairs = double(psi.N + 1) * (psi.M + 1);
+    bool from_pairs = with_S && pairs * pairs <= 3.0 * double(P) * P;
+    // The pairs give <O^* O'> - <O^*><O'> of uncentred sums, an error of eps (1 + |<O>|^2 / variance)
+    // where the Gram of the centred O has eps; so they serve only while no parameter's mean
+    // dominates.  fp64: mean squares up to the variances (a bit; 8 sites, 10 units, 2,048 samples in
+    // one chain against long double: 8e-15 and 9e-15 of the variance at a ratio of 0.9, 3.9e-14 and
+    // 7.8e-13 at 14).  fp32: up to 2e-13 of the variance, far below the fp32 rounding of O.
+    if (from_pairs)
+        launch_mean_dominated(t.Obar.p, t.diag.p, P, sizeof(T) == 8 ? 1.0 : 1024.0, t.sums.p + 4, S());
     // E, E2 and sum w go to page-locked memory; the host reads them, and <O> and F,
     // when they are asked for (the evaluation returns without synchronising, so a
     // solve that follows is queued behind it at once)
-    t.sums_host.ensure(4);
-    ANN_HIP_CHECK(hipMemcpyAsync(t.sums_host.p, t.sums.p, sizeof(double) * 4, hipMemcpyDeviceToHost, S()));
+    t.sums_host.ensure(5);
+    ANN_HIP_CHECK(hipMemcpyAsync(t.sums_host.p, t.sums.p, sizeof(double) * 5, hipMemcpyDeviceToHost, S()));
     t.sums_pending = true;
     t.of_pending = true;
+    if (from_pairs) ANN_HIP_CHECK(hipEventRecord(t.sums_ev.get(), S()));
+    // F = sum w conj(O) E_loc - E conj(<O>) (TDVP.cu.template:300) = sum w (E_loc - E) conj(O)
+    launch_weight_coef_centered_dev(s.w.p, s.e_loc.p, t.sums.p, n, coef.p, S());
+    structured_sums<T>(t, net, s.confs.p, s.words, g.p, 1, coef.p, n, t.Fd.p, 0.0, nullptr);
     t.confs.ensure(size_t(n) * s.words);
     ANN_HIP_CHECK(hipMemcpyAsync(t.confs.p, s.confs.p, sizeof(uint64_t) * n * s.words, hipMemcpyDeviceToDevice, S()));
     t.w.ensure(n);
@@ -1385,12 +1399,11 @@ void tdvp_eval_t(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with_S) {
     t.has_S = false;
     if (with_S) {
         t.S.ensure(size_t(P) * P);
-        // From the pairs of sites and pairs of units when nearly every (site, unit), the
-        // biases' constants included, carries a parameter: (N+1)^2 (M+1)^2 flop per sample
-        // against 4 P^2 for the Gram of the materialised O.  (They cross at a quarter of the
-        // pairs' count; the line is at a third, as the pairs' table has to be gathered.)
-        const double pairs = double(psi.N + 1) * (psi.M + 1);
-        if (pairs * pairs <= 3.0 * double(P) * P) {
+        if (from_pairs) {   // (F is computed meanwhile)
+            ANN_HIP_CHECK(hipEventSynchronize(t.sums_ev.get()));
+            from_pairs = t.sums_host.p[4] == 0.0;
+        }
+        if (from_pairs) {
             const SpinPlan plan = spin_plan(net.N, net.M, net.Mpad, n, true);
             if (!t.bits_valid) {
                 t.spin_bits.ensure(size_t(plan.bit_blocks) * plan.vpad);
@@ -1399,6 +1412,7 @@ void tdvp_eval_t(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with_S) {
             }
             t.gram_work.ensure(dense_gram_work_elems(psi.N, psi.M, n));
             t.gram_mean.ensure(P);
+            ScopedTimer route("gram_pairs", false);   // (counted only)
             ScopedTimer timer("gram");
             launch_dense_gram<T>(psi.layout, psi.N, psi.M, psi.Mpad, psi.kind == PSI_DEEP ? t.conn.p : nullptr,
                                  t.spin_bits.p, plan.vpad, g.p, s.w.p, n, P, t.gram_work.p, t.gram_mean.p, t.S.p, S());

@@ -448,6 +448,7 @@ struct Tdvp {
     bool kf_inverted = false;    // kf_Ci / kf_D hold the inverses for the current samples and kf_inv_shift
     double kf_inv_shift = 0.0;
     OwnedEvent fork_ev, join_ev, join2_ev;   // the evaluation's side-stream fork and joins
+    OwnedEvent sums_ev;                      // sums_host holds this evaluation's values
     // E, E2, wsum (sums_host) and O, F (from Obar, Fd) of the last evaluation are read
     // to the host on first use
     bool sums_pending = false, of_pending = false;
@@ -469,7 +470,7 @@ struct Tdvp {
     DevBuf<int> kf_idx;
     DevBuf<int> inv;            // inverse gather table [N][Mpad] (PsiDeep)
     DevBuf<double> dot_scratch;
-    DevBuf<double> sums;           // E.re, E.im, E2, sum w of the last evaluation
+    DevBuf<double> sums;           // E.re, E.im, E2, sum w, mean-dominated parameters of the last evaluation
     PinnedBuf<double> sums_host;
     DevBuf<cplx<double>> coef;     // per-sample weights of the statistics
     // materialised O [count][P] of wave functions without a structured O (PsiCNN)

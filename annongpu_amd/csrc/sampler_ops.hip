@@ -229,6 +229,24 @@ __global__ void sr_diag_kernel(int layout, int N, int M, int Mpad, const double*
     (void)Mpad;
 }
 
+// out = number of parameters whose |<O>|^2 exceeds limit times their variance (or is not a number)
+__global__ __launch_bounds__(1024) void mean_dominated_kernel(const cplx<double>* Obar, const double* diag, int P,
+                                                              double limit, double* out) {
+    __shared__ int sh[16];
+    int n = 0;
+    for (int k = threadIdx.x; k < P; k += 1024) {
+        const cplx<double> o = Obar[k];
+        if (!(o.re * o.re + o.im * o.im <= limit * diag[k])) n++;
+    }
+    for (int d = 32; d > 0; d >>= 1) n += __shfl_xor(n, d);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; w++) n += sh[w];
+        *out = double(n);
+    }
+}
+
 // S += alpha * conj(o) o^T
 __global__ void rank1_kernel(cplx<double>* S, const cplx<double>* o, int P, double alpha) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -344,6 +362,12 @@ void launch_precond(cplx<double>* z, const cplx<double>* r, const double* diag, 
 void launch_sr_diag(int layout, int N, int M, int Mpad, const double* wsum, const cplx<double>* Dj,
                     const cplx<double>* Obar, int P, double* diag, hipStream_t stream) {
     sr_diag_kernel<<<blocks_for(P), 256, 0, stream>>>(layout, N, M, Mpad, wsum, Dj, Obar, P, diag);
+    ANN_LAUNCH_CHECK();
+}
+
+void launch_mean_dominated(const cplx<double>* Obar, const double* diag, int P, double limit, double* out,
+                           hipStream_t stream) {
+    mean_dominated_kernel<<<1, 1024, 0, stream>>>(Obar, diag, P, limit, out);
     ANN_LAUNCH_CHECK();
 }
 

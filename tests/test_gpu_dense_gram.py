@@ -3,7 +3,11 @@ edges of the kernel's tiles (64 site pairs a wave, 32 unit pairs, 16 samples a s
 words) and over the layouts that reach it, sample counts and weights that do not sum to one.
 
 The O_k samples are exact copies of what S is built from, so both sides are fp64 sums of the
-same products: |S - S_ref| <= 4 n eps max|sum w |O_k|^2| entrywise (n summands)."""
+same products: |S - S_ref| <= 4 n eps max|sum w |O_k|^2| entrywise (n summands).
+
+The pairs serve while no parameter's squared mean exceeds its variance (fp32: 1,024 times it); where
+one does, S comes from the centred O_k and its error stays within the rounding of the n products and
+of the centring, relative to the two parameters' spreads."""
 import numpy as np
 import pytest
 
@@ -27,6 +31,24 @@ def net(kind, N, M, rng):
     return A.PsiDeep(N, gauss(N, 0.1), [gauss(M, 0.1)], [conn], [gauss(conn.shape, 0.2)], 1.0 + rng.random(M))
 
 
+def evaluate(A, psi, op, ens):
+    """the TDVP object and whether its S came from pairs"""
+    t = A.TDVP(psi.num_params)
+    A.profiler_reset()
+    A.start_profiling()
+    t.eval(op, psi, ens)
+    A.stop_profiling()
+    assert A.profiler_query("gram")[1] == 1
+    return t, A.profiler_query("gram_pairs")[1] == 1
+
+
+def dominance(O, w):
+    """largest ratio of a squared mean to the variance (inf where there is no variance)"""
+    m = np.abs(w @ O) ** 2
+    d = w @ np.abs(O) ** 2 - m
+    return np.where(d > 0, m / np.where(d > 0, d, 1), np.inf).max()
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 @pytest.mark.parametrize("kind,N,M,n", [("circulant", 1, 1, 1), ("circulant", 11, 6, 65), ("rbm", 11, 7, 64),
                                         ("rbm", 12, 24, 1000), ("shuffled", 23, 9, 129), ("circulant", 22, 8, 15),
@@ -41,12 +63,47 @@ def test_dense_gram(kind, N, M, n, precision):
     if N % 64:
         confs[:, -1] &= np.uint64(2 ** (N % 64) - 1)
     w = rng.random(n) / n
-    t = A.TDVP(psi.num_params)
-    t.eval(A.Operator(1.0 * A.sigma_z(0)), psi, A.SampleList(N, confs, w))
+    t, pairs = evaluate(A, psi, A.Operator(1.0 * A.sigma_z(0)), A.SampleList(N, confs, w))
     O = t.O_k_samples
+    if n > 1:
+        assert pairs == (dominance(O, w) <= (1 if precision == "fp64" else 1024))
     mean = w @ O
     S = (O.conj() * w[:, None]).T @ O - np.outer(mean.conj(), mean)
     assert np.abs(t.S_matrix - S).max() <= 4 * max(n, 8) * np.finfo(float).eps * (w @ np.abs(O) ** 2).max()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("bias,flips", [(0.0, 0.5), (0.0, 0.02), (0.8, 0.5), (0.8, 0.02)])
+def test_dominating_means(bias, flips, precision):
+    """hidden biases far above the spread of the angles and polarised spins; n a power of two, so that
+    the weights sum to one exactly.  Per entry, in units of the two spreads: n products and sums of
+    eps (8 for the complex parts), the centring's eps |O| and, in fp32, its rounding of the centred O.
+    (From uncentred sums the error is eps |O|^2, 1e5 to 1e6 in these units.)"""
+    import annongpu_amd as A
+    N, M, n = 12, 24, 512
+    rng = np.random.default_rng(3)
+    conn = (np.arange(M)[None, :] + np.arange(N)[:, None]) % N
+    W = 1e-3 * (rng.standard_normal((N, M)) + 1j * rng.standard_normal((N, M)))
+    psi = A.PsiDeep(N, np.zeros(N), [bias * (1 + 0.1 * rng.random(M))], [conn], [W], np.ones(M))
+    psi.precision = precision
+    bits = rng.random((n, N)) >= flips
+    confs = (bits.astype(np.uint64) << np.arange(N, dtype=np.uint64)).sum(1, dtype=np.uint64)[:, None]
+    t, pairs = evaluate(A, psi, A.Operator(1.0 * A.sigma_z(0)), A.SampleList(N, confs))
+    O = t.O_k_samples.astype(np.clongdouble)
+    w = np.full(n, 1 / n)
+    ratio = dominance(O.astype(complex), w)
+    assert pairs == (ratio <= (1 if precision == "fp64" else 1024))
+    x = O - O.mean(0)
+    S = (x.conj().T @ x) / n
+    spread = np.sqrt(np.diag(S).real)
+    size = np.sqrt((np.abs(O) ** 2).mean(0)) / spread
+    eps = np.finfo(float).eps
+    bound = 8 * (n + 3) * eps + 4 * eps * (size[:, None] + size[None, :])
+    if pairs:
+        bound = bound + 8 * (n + 3) * eps * size[:, None] * size[None, :]
+    elif precision == "fp32":
+        bound = bound + 4 * np.finfo(np.float32).eps
+    assert np.all(np.abs(t.S_matrix - S) <= bound * spread[:, None] * spread[None, :])
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
