@@ -1403,19 +1403,21 @@ void tdvp_eval_t(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with_S) {
             ANN_HIP_CHECK(hipEventSynchronize(t.sums_ev.get()));
             from_pairs = t.sums_host.p[4] == 0.0;
         }
-        if (from_pairs) {
+        // (the pairs' table takes a quarter of S, O n P values: where the former does not fit, the
+        // latter may)
+        if (from_pairs && t.chol.try_ensure((dense_gram_work_elems(psi.N, psi.M, n) + 1) / 2)) {
             const SpinPlan plan = spin_plan(net.N, net.M, net.Mpad, n, true);
             if (!t.bits_valid) {
                 t.spin_bits.ensure(size_t(plan.bit_blocks) * plan.vpad);
                 launch_spin_bits(s.confs.p, s.words, n, net.N, plan.vpad, t.spin_bits.p, S());
                 t.bits_valid = true;
             }
-            t.gram_work.ensure(dense_gram_work_elems(psi.N, psi.M, n));
             t.gram_mean.ensure(P);
             ScopedTimer route("gram_pairs", false);   // (counted only)
             ScopedTimer timer("gram");
             launch_dense_gram<T>(psi.layout, psi.N, psi.M, psi.Mpad, psi.kind == PSI_DEEP ? t.conn.p : nullptr,
-                                 t.spin_bits.p, plan.vpad, g.p, s.w.p, n, P, t.gram_work.p, t.gram_mean.p, t.S.p, S());
+                                 t.spin_bits.p, plan.vpad, g.p, s.w.p, n, P, reinterpret_cast<double*>(t.chol.p),
+                                 t.gram_mean.p, t.S.p, S());
         } else {
             DevBuf<cplx<T>> O;
             O.ensure(size_t(n) * P);
@@ -1423,10 +1425,10 @@ void tdvp_eval_t(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with_S) {
                 ScopedTimer timer("o_k");
                 launch_materialize_ok<T>(net, s.confs.p, s.words, g.p, n, t.Obar.p, O.p, S());
             }
-            t.gram_part.ensure(gram_work_elems(P, n));
+            t.chol.ensure(gram_work_elems(P, n));
             {
                 ScopedTimer timer("gram");
-                launch_gram<T>(O.p, s.w.p, n, P, t.gram_part.p, t.S.p, S());
+                launch_gram<T>(O.p, s.w.p, n, P, t.chol.p, t.S.p, S());
             }
             // reference S = sum w conj(O) O - conj(<O>) <O>; with centred O this needs
             // (1 - sum w) conj(<O>) <O> added back (zero for normalised weights)
@@ -1521,10 +1523,10 @@ void tdvp_eval_generic(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with
     t.has_S = false;
     if (with_S) {
         t.S.ensure(size_t(P) * P);
-        t.gram_part.ensure(gram_work_elems(P, n));
+        t.chol.ensure(gram_work_elems(P, n));
         {
             ScopedTimer timer("gram");
-            launch_gram<T>(O.p, s.w.p, n, P, t.gram_part.p, t.S.p, S());
+            launch_gram<T>(O.p, s.w.p, n, P, t.chol.p, t.S.p, S());
         }
         // S = sum w conj(O) O - conj(<O>) <O>
         launch_rank1(t.S.p, t.Obar.p, P, -1.0, S());

@@ -48,6 +48,18 @@ struct DevBuf {
         ANN_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&p), sizeof(T) * (m > 0 ? m : 1)));
         n = m;
     }
+    // the same, but false (and an empty buffer) where the memory is not there
+    bool try_ensure(size_t m) {
+        if (m <= n && p) return true;
+        release();
+        if (hipMalloc(reinterpret_cast<void**>(&p), sizeof(T) * (m > 0 ? m : 1)) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+            return false;
+        }
+        n = m;
+        return true;
+    }
     // ordered after the work already queued on the library stream; returns when done
     void upload(const T* h, size_t m) {
         ensure(m);
@@ -403,11 +415,12 @@ struct Tdvp {
     std::vector<cd> O, F;
     bool has_S = false, has_samples = false;
     DevBuf<cplx<double>> S, Obar, Fd;
-    DevBuf<cplx<double>> chol, chol_work;   // Cholesky factor of the scaled S + shift and its panel workspace
+    // Cholesky factor of the scaled S + shift, and before the solve the workspace S is built in
+    // (the pairs' table, the sample chunks of the other Gram)
+    DevBuf<cplx<double>> chol;
+    DevBuf<cplx<double>> chol_work;         // the factorisation's block inverses
     DevBuf<double> chol_dinv;               // the diagonal scaling of that factor
-    DevBuf<double> gram_work;               // pair products of a dense net's S (gram_dense.hip)
     DevBuf<cplx<double>> gram_mean;
-    DevBuf<cplx<double>> gram_part;         // sample chunks of the Gram of a materialised O
     // structured O of the last evaluation (dense nets)
     int precision = 0, words = 0, N = 0, M = 0, Mpad = 0, C = 0, layout = 0, npad = 0;
     int64_t count = 0;

@@ -8,6 +8,8 @@ same products: |S - S_ref| <= 4 n eps max|sum w |O_k|^2| entrywise (n summands).
 The pairs serve while no parameter's squared mean exceeds its variance (fp32: 1,024 times it); where
 one does, S comes from the centred O_k and its error stays within the rounding of the n products and
 of the centring, relative to the two parameters' spreads."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -104,6 +106,73 @@ def test_dominating_means(bias, flips, precision):
     elif precision == "fp32":
         bound = bound + 4 * np.finfo(np.float32).eps
     assert np.all(np.abs(t.S_matrix - S) <= bound * spread[:, None] * spread[None, :])
+
+
+def ring(N, M, n):
+    import annongpu_amd as A
+    rng = np.random.default_rng(5)
+    psi = net("circulant", N, M, rng)
+    psi.precision = "fp32"
+    confs = rng.integers(0, 2 ** 63, size=(n, 1), dtype=np.uint64) >> np.uint64(max(0, 63 - N))
+    return A, psi, A.Operator(1.0 * A.sigma_z(0)), A.SampleList(N, confs)
+
+
+def free_memory(A):
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert A._lib.lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_memory_held():
+    """after an evaluation and a solve the object holds S and the factor, and no third buffer of their
+    size class: the workspace of S is the factor's (72 MB of pairs here)"""
+    A, psi, op, ens = ring(4, 3, 8)
+    evaluate(A, psi, op, ens)[0].solve(1e-2, "cholesky")   # streams, code and their memory
+    A, psi, op, ens = ring(32, 128, 256)
+    P = psi.num_params
+    A.log_psi(psi, ens)
+    before = free_memory(A)
+    t, pairs = evaluate(A, psi, op, ens)
+    t.solve(1e-2, "cholesky")
+    held = before - free_memory(A)
+    assert held <= 2 * 16 * P * P + 48 * 2 ** 20
+    assert pairs
+
+
+def test_pairs_do_not_fit():
+    """S next to the samples' O fits the card, S next to the pairs' table does not: the evaluation
+    still answers"""
+    A, psi, op, ens = ring(62, 200, 64)   # S 2.6 GB, the table 0.64 GB, O 6 MB
+    P = psi.num_params
+    t, pairs = evaluate(A, psi, op, ens)
+    assert pairs
+    want = t.S_matrix[:100].copy()
+    diag = np.diag(t.S_matrix).real.copy()
+    del t
+    hip = A._lib.lib
+
+    def allocate(size):
+        p = ctypes.c_void_p()
+        return p if hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(size)) == 0 else None
+
+    room = allocate(16 * P * P + 350 * 2 ** 20)
+    size, held = 2 ** 36, []
+    while size >= 2 ** 24:
+        p = allocate(size)
+        if p:
+            held.append(p)
+        else:
+            size //= 2
+    hip.hipGetLastError()
+    assert hip.hipFree(room) == 0
+    try:
+        t, pairs = evaluate(A, psi, op, ens)
+    finally:
+        for p in held:
+            assert hip.hipFree(p) == 0
+    assert not pairs
+    d = np.sqrt(diag)
+    assert np.abs((t.S_matrix[:100] - want) / d / d[:100, None]).max() <= 1e-5
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
