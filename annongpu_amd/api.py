@@ -1260,9 +1260,12 @@ class TDVP:
             self._h = None
 
     def eval(self, op, psi, ensemble):
+        """E, F, <O> and S on the ensemble; may return before the device is done (reading a result
+        waits for it)"""
         check(lib.ann_tdvp_eval(self._h, op._h, psi._h, ensemble._h, 1))
 
     def eval_F(self, op, psi, ensemble):
+        """eval without S"""
         check(lib.ann_tdvp_eval(self._h, op._h, psi._h, ensemble._h, 0))
 
     @property

@@ -245,7 +245,10 @@ int ann_kl_set_log_psi_scale(ann_kl kl, double scale);
 /* TDVP(num_params, gpu) -- network_functions/TDVP.hpp:16-101, MAIN:465-489 */
 int ann_tdvp_create(ann_tdvp* out, uint32_t num_params);
 int ann_tdvp_destroy(ann_tdvp tdvp);
-/* eval (with_S = 1) and eval_F (with_S = 0) -- TDVP.cu.template:181-334 */
+/* eval (with_S = 1) and eval_F (with_S = 0) -- TDVP.cu.template:181-334.  Either may return with
+ * its work, S included, still queued on the device: a time taken around the call alone is not the
+ * evaluation's.  psi, op and ens may be changed or destroyed at once; what the evaluation read of
+ * them is ordered before. */
 int ann_tdvp_eval(ann_tdvp tdvp, ann_operator op, ann_psi psi, ann_ensemble ens, int32_t with_S);
 /* S_matrix [P][P], F_vector, O_k_vector, E_local, E2_local, var_H (MAIN:467-474) */
 int ann_tdvp_get_S(ann_tdvp tdvp, double* S);

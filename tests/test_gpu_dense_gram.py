@@ -175,6 +175,34 @@ def test_pairs_do_not_fit():
     assert np.abs((t.S_matrix[:100] - want) / d / d[:100, None]).max() <= 1e-5
 
 
+@pytest.mark.parametrize("bias", [0.1, 0.8])
+def test_next_calls_leave_S_alone(bias):
+    """an evaluation may return with S still queued (a few ms of work here): the same wave function and
+    ensemble changed, evaluated elsewhere and destroyed meanwhile do not reach it"""
+    A, psi, op, _ = ring(62, 200, 256)
+    psi.precision = "fp64"
+    if bias > 0.5:   # the means dominate: S from the centred samples
+        psi.params = np.concatenate([np.zeros(62), np.full(200, bias), 1e-3 * psi.params[262:]])
+    first = psi.params
+
+    def chains():
+        ens = A.MonteCarloSpins(256, 2, 3, 256, seed=4, persistent=True)
+        A.log_psi(psi, ens)
+        return ens
+
+    t, pairs = evaluate(A, psi, op, chains())
+    assert pairs == (bias < 0.5)
+    want = t.S_matrix[:300].copy()
+    for _ in range(2):
+        psi.params = first
+        ens = chains()
+        t.eval(op, psi, ens)
+        psi.params = 0.5 * first
+        A.TDVP(psi.num_params).eval_F(op, psi, ens)
+        del ens
+        assert np.array_equal(t.S_matrix[:300], want)
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 @pytest.mark.parametrize("n", [1, 127, 129, 300, 1025])
 def test_gram_of_materialised_samples(n, precision):
