@@ -53,12 +53,6 @@ __device__ void build_lut(const CnnPair<T>& f, const cplx<T>* params, cplx<T>* l
     }
 }
 
-// orders a wave's LDS accesses (other lanes read what a lane wrote)
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 __device__ __forceinline__ uint16_t pattern_of(const int* nbr0, int v0, const uint64_t (&w)[kMaxWords], int x) {
     int p = 0;
     for (int k = 0; k < v0; k++) {

@@ -200,6 +200,14 @@ __device__ inline void flip_bit(uint64_t* m, int i) {
     for (int k = 0; k < kMaxWords; k++) m[k] ^= b & (uint64_t(0) - uint64_t(k == (i >> 6)));
 }
 
+// orders a wave's LDS accesses where lanes read what other lanes wrote: the hardware keeps
+// their order, but nothing else keeps the compiler from moving a lane's load above its own store
+// to another address
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // ------------------------------------------------------ wave reductions
 // GFX9 DPP all-reduce: quad_perm [1,0,3,2] and [2,3,0,1], row_half_mirror and
 // row_mirror give 16-lane row sums, row_bcast:15 / row_bcast:31 fold the four

@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kEThreads, 4) void local_energy_terms_kernel(
     // off-diagonal groups with a coefficient, in group order
     for (int sl = wave; sl < samples; sl += kEWaves) {
         if (lane < kMaxWords) cw[sl * kMaxWords + lane] = lane < words ? confs[(s0 + sl) * words + lane] : 0;
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         const uint64_t* c = cw + sl * kMaxWords;
         double2 d = {0.0, 0.0};
         if (op.diag_group >= 0)

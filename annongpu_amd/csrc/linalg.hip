@@ -364,6 +364,7 @@ __global__ __launch_bounds__(256) void potrf_inv_kernel(const cplx<double>* A, i
         }
 #pragma unroll
         for (int q = 0; q < 4; q++) ysh[w][q][lane] = y[q];
+        wave_sync();
         // operands of A_rc -= sum_q L_r,j0+q y_qc (L_r,j0+q = conj(y_qr), rows below the block)
         const double2 yr = ysh[w][lk][16 * w + lc];
         const bool below = 16 * w + lc > j0 + 3;
