@@ -119,7 +119,6 @@ struct PairTables {
     uint32_t* aff0;   // [N][n0] site | toggled pattern bits << 8
     uint8_t* nbr1;    // [N][v1]
     uint8_t* aff1;    // [N][n1] sites in increasing order
-    size_t bytes;
     __device__ PairTables(const CnnPair<T>& f, unsigned char* smem) {
         lut = reinterpret_cast<cplx<T>*>(smem);
         aff0 = reinterpret_cast<uint32_t*>(lut + (size_t(f.C0) << f.v0));
@@ -678,6 +677,7 @@ bool cnn_pair_log_psi(const CnnView<T>& v, const uint64_t* confs, int words, int
                                                                          count, lp, log_psi, weight);
     });
     ANN_LAUNCH_CHECK();
+    count_route("cnn_pair_log_psi");
     return true;
 }
 
@@ -706,6 +706,7 @@ bool cnn_pair_mc(const CnnView<T>& v, uint64_t* chain_confs, int words, int num_
             run(cnn_pair_mc_kernel<T, decltype(cb)::value, decltype(vm)::value, 64>);
     });
     ANN_LAUNCH_CHECK();
+    count_route("cnn_pair_mc");
     return true;
 }
 
@@ -730,6 +731,7 @@ bool cnn_pair_local_energy(const CnnView<T>& v, const OpView& op, const uint64_t
             run(cnn_pair_local_energy_kernel<T, decltype(cb)::value, decltype(vm)::value, 64>);
     });
     ANN_LAUNCH_CHECK();
+    count_route("cnn_pair_local_energy");
     return true;
 }
 
@@ -746,6 +748,7 @@ bool cnn_pair_ok(const CnnView<T>& v, const uint64_t* confs, int words, int64_t 
                                                                    v.num_params, O);
     });
     ANN_LAUNCH_CHECK();
+    count_route("cnn_pair_ok");
     return true;
 }
 

@@ -334,6 +334,7 @@ void launch_local_energy_terms(const DenseView<float>& net, const OpView& op, co
     else
         pick_words(std::false_type{});
     ANN_LAUNCH_CHECK();
+    count_route("local_energy_terms");
 }
 
 }  // namespace ann

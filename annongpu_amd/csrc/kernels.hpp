@@ -87,6 +87,9 @@ struct PauliOpView {
 // ---------------------------------------------------------------- launches
 // Every wrapper launches on `stream` and throws HipError on a launch failure.
 
+// counts a launch under name while the profiler runs (which kernels served a call)
+void count_route(const char* name);
+
 void launch_enumerate_confs(uint64_t* confs, int64_t first_index, int64_t count, int words,
                             hipStream_t stream);
 // Pauli strings by index (PauliString::enumerate, PauliString.hpp:30-35): site i takes

@@ -105,6 +105,10 @@ void Runtime::collect() {
 
 hipStream_t lib_stream() { return Runtime::get().stream(); }
 
+void count_route(const char* name) {
+    if (Runtime::get().profiling) Runtime::get().untimed[name]++;
+}
+
 static hipStream_t S() { return Runtime::get().stream(); }
 
 // --------------------------------------------------------------------- Psi
@@ -1413,7 +1417,7 @@ void tdvp_eval_t(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with_S) {
                 t.bits_valid = true;
             }
             t.gram_mean.ensure(P);
-            ScopedTimer route("gram_pairs", false);   // (counted only)
+            count_route("gram_pairs");
             ScopedTimer timer("gram");
             launch_dense_gram<T>(psi.layout, psi.N, psi.M, psi.Mpad, psi.kind == PSI_DEEP ? t.conn.p : nullptr,
                                  t.spin_bits.p, plan.vpad, g.p, s.w.p, n, P, reinterpret_cast<double*>(t.chol.p),

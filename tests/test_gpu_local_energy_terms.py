@@ -74,7 +74,11 @@ def test_local_energy_terms(kind, N, M, n, real_f, precision):
     bits[:, :N] = spins > 0
     confs = np.ascontiguousarray(np.packbits(bits, axis=1, bitorder="little")).view(np.uint64)
     H = operator(A, kind, N, rng)
+    A.profiler_reset()
+    A.start_profiling()
     e = A.local_energies(A.Operator(H), psi, A.SampleList(N, confs))
+    A.stop_profiling()
+    assert A.profiler_query("local_energy_terms")[1] == (precision == "fp32" and kind != "three")
     ref, size = reference(H, spins @ W + b, W, f, spins)
     tol = 1e-12 if precision == "fp64" else 8 * np.finfo(np.float32).eps * (M + 1)
     assert np.all(np.abs(e - ref) <= tol * size)
