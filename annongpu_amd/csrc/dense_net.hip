@@ -302,7 +302,7 @@ __global__ __launch_bounds__(kBlock) void mc_sweep_kernel(DenseView<T> net, uint
 }
 
 // E_loc(s) = sum_groups coef_g(s) * psi(s')/psi(s)  (Operator.hpp:36-121), any strings (in
-// fp32 those that flip at most two sites are served by eloc_dense.hip)
+// fp32 most that flip at most two sites are served by eloc_dense.hip)
 template <typename T, int U>
 __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? 4 : 1) void local_energy_kernel(DenseView<T> net, OpView op,
                                                               const uint64_t* confs,
@@ -652,7 +652,7 @@ void launch_local_energy(const DenseView<T>& net, const OpView& op, const uint64
                          const cplx<T>* theta, int64_t count, cplx<double>* e_loc, hipStream_t stream) {
     if (count <= 0) return;
     if constexpr (sizeof(T) == 4) {
-        if (local_energy_terms_supported(op)) {
+        if (local_energy_terms_serves(net.M, op, count)) {
             launch_local_energy_terms(net, op, confs, theta, count, e_loc, stream);
             return;
         }

@@ -20,11 +20,13 @@
 // [unit][site], and its samples' 2 theta, C1, C2 in LDS: per unit a lane reads its sites'
 // entries (4 x 8 bytes) and the sample's 24 bytes once for its two terms.  The unit sums are
 // taken per tile in fp32 and over the tiles in fp64.
-// 10x10 Heisenberg, 400 units, 16,384 samples, fp32: 1,205 -> 565 us.
+// 10x10 Heisenberg, 400 units, 16,384 samples, fp32: 1,205 -> 565 us.  With few terms for the units
+// the general kernel is the faster one: local_energy_terms_serves.
 #include "kernels.hpp"
 #include "wave_net.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace ann {
@@ -288,30 +290,68 @@ __global__ __launch_bounds__(kEThreads, 4) void local_energy_terms_kernel(
 
 }  // namespace
 
-// log2 of the units per tile, 32 at most and 4 at least, whose D fit the tile (-1: too many terms)
-static int eloc_units_log2(const OpView& op) {
-    const int64_t entries = std::max<int64_t>(1, int64_t(op.num_groups) * (op.equal_spins ? 2 : 1));
-    int l = 5;
-    while (l >= 2 && (entries << l) * int64_t(sizeof(Pair)) > kETile) l--;
-    return l >= 2 ? l : -1;
+namespace {
+
+struct TermsPlan {
+    int units = 0;       // log2 of the units per tile, 32 at most and 4 at least, whose D fit the tile
+    int per_block = 0;   // samples per workgroup
+    size_t lds = 0;
+};
+
+// false: too many terms
+bool terms_plan(const OpView& op, int64_t count, TermsPlan* p) {
+    const int G = std::max(op.num_groups, 1);
+    const int entries = op.equal_spins ? 2 * G : G;
+    if (op.max_flips > 2 || G > kEList) return false;
+    p->units = 5;
+    while (p->units >= 2 && (int64_t(entries) << p->units) * int64_t(sizeof(Pair)) > kETile) p->units--;
+    if (p->units < 2) return false;
+    // as many samples per workgroup as pay for its tile, fewer where that would leave CUs
+    // without their two workgroups, and no more than the term list holds
+    const int64_t want = std::min<int64_t>(kEThreads / 32, (count + 511) / 512);
+    p->per_block = int(std::min<int64_t>(want, std::max(1, kEList / G)));
+    p->lds = eloc_tile_bytes(kEThreads, p->per_block, 1 << p->units, entries) + sizeof(double2) * p->per_block +
+             sizeof(uint64_t) * p->per_block * kMaxWords + sizeof(int) * (2 * p->per_block + 1) +
+             sizeof(uint16_t) * size_t(p->per_block) * G;
+    return true;
 }
 
-bool local_energy_terms_supported(const OpView& op) {
-    return op.max_flips <= 2 && op.num_groups <= kEList && eloc_units_log2(op) >= 0;
+}  // namespace
+
+// The kernel's time is that of its rounds of workgroups, each a walk over the units per 2,048 terms:
+// 0.05 us a unit, 4 us a tile, and the terms' own operations; an operator with few terms leaves
+// most of its lanes idle.  The general kernel's is that of its chain of groups (0.8 us a group of up
+// to 64 units, more for more units; beyond 512 its registers spill), or of its waves in turn where
+// the samples fill the chip.  So: whichever is the shorter by this estimate, fitted to 1,327
+// measurements of both (3 to 1,596 groups, 2 to 1,000 units, 1 to 65,536 samples); the one it takes
+// is the faster within 5 % for all but 31 of them, within 10 % for all but 15.
+// 448 units, 4,000 samples, us here and there: 4 fields 92 and 15, 36 fields 106 and 72, 100 fields
+// 170 and 203, 100 bonds 136 and 186; 16,384 samples, 780 pairs of 40 sites, 128 units 1,166 and 2,583,
+// 448 units 3,540 and 3,432; 1,596 pairs, 448 units 13,732 and 6,753.
+bool local_energy_terms_serves(int M, const OpView& op, int64_t count) {
+    TermsPlan p;
+    if (!terms_plan(op, count, &p)) return false;
+    const int64_t blocks = (count + p.per_block - 1) / p.per_block;
+    const int64_t resident = 256 * (p.lds > 80 * 1024 ? 1 : 2);
+    const double rounds = double((blocks + resident - 1) / resident);
+    const double terms = double(op.terms) * p.per_block;
+    const double passes = std::ceil(terms / (2 * kERounds * kEThreads));
+    const double here = rounds * (12.5 + M * (passes * (0.048 + 4.0 / (1 << p.units)) + 0.00015 * terms));
+    int lane_units = 1;   // units per lane of the general kernel
+    for (int u : {1, 2, 4, 7, 8, 16})
+        if ((M + 63) / 64 <= (lane_units = u)) break;
+    const double wide = lane_units <= 8 ? 1.0 + 0.064 * (lane_units - 1) : 5.3;
+    const double general = 4.8 + op.num_groups * wide * std::max(0.78, 0.256e-3 * double(count));
+    return here < general;
 }
 
 void launch_local_energy_terms(const DenseView<float>& net, const OpView& op, const uint64_t* confs,
                                const cplx<float>* theta, int64_t count, cplx<double>* e_loc, hipStream_t stream) {
     if (count <= 0) return;
-    const int G = std::max(op.num_groups, 1);
-    // as many samples per workgroup as pay for its tile, fewer where that would leave CUs
-    // without their two workgroups, and no more than the term list holds
-    const int64_t want = std::min<int64_t>(kEThreads / 32, (count + 511) / 512);
-    const int per_block = int(std::min<int64_t>(want, std::max(1, kEList / G)));
-    const int units = eloc_units_log2(op), entries = op.equal_spins ? 2 * G : G;
-    const size_t lds = eloc_tile_bytes(kEThreads, per_block, 1 << units, entries) + sizeof(double2) * per_block +
-                       sizeof(uint64_t) * per_block * kMaxWords + sizeof(int) * (2 * per_block + 1) +
-                       sizeof(uint16_t) * size_t(per_block) * G;
+    TermsPlan plan;
+    if (!terms_plan(op, count, &plan)) throw std::invalid_argument("local energies: too many terms");
+    const int per_block = plan.per_block, units = plan.units;
+    const size_t lds = plan.lds;
     auto pick = [&](auto realf, auto words) {
         auto kernel = local_energy_terms_kernel<decltype(realf)::value, decltype(words)::value>;
         if (lds > 64 * 1024)

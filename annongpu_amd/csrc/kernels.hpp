@@ -74,6 +74,7 @@ struct OpView {
     int diag_group;                  // the group without flips (-1: none)
     int max_flips;                   // most sites any group flips
     int equal_spins;                 // a group of two sites may have a coefficient where their spins are equal
+    float terms;                     // off-diagonal groups with a coefficient in random spins, on average
 };
 
 // Pauli-sum operator acting on Pauli-string configurations (string n maps x to
@@ -126,8 +127,9 @@ void launch_mc_sweep(const DenseView<T>& net, uint64_t* chain_confs, cplx<T>* th
                      int words, int move, int64_t num_proposals, uint64_t counter, uint64_t seed,
                      uint32_t* accepted, hipStream_t stream);
 
-// E_loc of the operators local_energy_terms_supported accepts, fp32 (eloc_dense.hip)
-bool local_energy_terms_supported(const OpView& op);
+// fp32 E_loc of operators whose strings flip at most two sites (eloc_dense.hip), and whether that
+// kernel is the one for the net, the operator and the number of samples
+bool local_energy_terms_serves(int M, const OpView& op, int64_t count);
 void launch_local_energy_terms(const DenseView<float>& net, const OpView& op, const uint64_t* confs,
                                const cplx<float>* theta, int64_t count, cplx<double>* e_loc, hipStream_t stream);
 

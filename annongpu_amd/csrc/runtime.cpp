@@ -807,6 +807,8 @@ const DeviceOp& Operator::device(int words) {
         }
         if (up != 0.0 || down != 0.0) d->equal_spins = true;
     }
+    for (size_t g = 0; g < groups.size(); g++)
+        if (int(g) != d->diag_group) d->terms += sites[2 * g + 1] >= 0 && !d->equal_spins ? 0.5f : 1.0f;
     d->group_flip.upload(flip.data(), flip.size());
     d->group_begin.upload(begin.data(), begin.size());
     d->string_zy.upload(zy.data(), zy.size());

@@ -300,10 +300,11 @@ struct DeviceOp {
     DevBuf<int> group_begin, group_sites;
     int diag_group = -1, max_flips = 0;
     bool equal_spins = false;
+    float terms = 0.0f;
     DevBuf<double> string_coef;
     OpView view() const {
         return {num_groups, words, group_flip.p, group_begin.p, string_zy.p, string_coef.p, group_sites.p, diag_group,
-                max_flips, equal_spins ? 1 : 0};
+                max_flips, equal_spins ? 1 : 0, terms};
     }
 };
 
