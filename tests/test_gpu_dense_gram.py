@@ -123,6 +123,20 @@ def free_memory(A):
     return free.value
 
 
+@pytest.mark.parametrize("n,expected", [(64, False), (512, True)])
+def test_few_samples_of_many_parameters(n, expected):
+    """few samples do not pay for the pairs' table of 12,662 parameters; bound as above"""
+    A, psi, op, ens = ring(62, 200, n)
+    t, pairs = evaluate(A, psi, op, ens)
+    assert pairs == expected
+    O = t.O_k_samples
+    x = O - O.mean(0)
+    rows = np.r_[0:3, 61, 62, 261, 262, 5000, 12661]
+    S = x[:, rows].conj().T @ x / n
+    eps = np.finfo(float).eps if expected else np.finfo(np.float32).eps   # (the centred O is rounded)
+    assert np.abs(t.S_matrix[rows] - S).max() <= 4 * max(n, 8) * eps * (np.abs(O) ** 2).mean(0).max()
+
+
 def test_memory_held():
     """after an evaluation and a solve the object holds S and the factor, and no third buffer of their
     size class: the workspace of S is the factor's (72 MB of pairs here)"""
@@ -142,7 +156,7 @@ def test_memory_held():
 def test_pairs_do_not_fit():
     """S next to the samples' O fits the card, S next to the pairs' table does not: the evaluation
     still answers"""
-    A, psi, op, ens = ring(62, 200, 64)   # S 2.6 GB, the table 0.64 GB, O 6 MB
+    A, psi, op, ens = ring(62, 200, 512)   # S 2.6 GB, the table 0.64 GB, O 52 MB
     P = psi.num_params
     t, pairs = evaluate(A, psi, op, ens)
     assert pairs
@@ -179,14 +193,14 @@ def test_pairs_do_not_fit():
 def test_next_calls_leave_S_alone(bias):
     """an evaluation may return with S still queued (a few ms of work here): the same wave function and
     ensemble changed, evaluated elsewhere and destroyed meanwhile do not reach it"""
-    A, psi, op, _ = ring(62, 200, 256)
+    A, psi, op, _ = ring(62, 200, 512)
     psi.precision = "fp64"
     if bias > 0.5:   # the means dominate: S from the centred samples
         psi.params = np.concatenate([np.zeros(62), np.full(200, bias), 1e-3 * psi.params[262:]])
     first = psi.params
 
     def chains():
-        ens = A.MonteCarloSpins(256, 2, 3, 256, seed=4, persistent=True)
+        ens = A.MonteCarloSpins(512, 2, 3, 512, seed=4, persistent=True)
         A.log_psi(psi, ens)
         return ens
 
