@@ -129,17 +129,18 @@ __device__ inline int64_t xcd_tile(int64_t b, int64_t n) {
 // ------------------------------------------------------------------ Gram
 // S[k][k'] = sum_s w_s conj(O_sk) O_sk' for the upper-triangular tile pairs, mirrored
 // into the lower triangle; samples are the k of the product, 16 per stage, staged in
-// LDS double-buffered with the next stage's global loads in flight during the MFMAs.  With
-// part, workgroup (tile, z) takes the samples of chunk z and leaves its tile there
-// ([chunk][tile][64][64]) for gram_finish_kernel.
-template <typename T>
+// LDS double-buffered with the next stage's global loads in flight during the MFMAs.  SPLIT:
+// workgroup (tile, z) takes the samples of chunk z and leaves its tile in out
+// ([chunk][tile][64][64]) for gram_finish_kernel; else out is S.  (With the choice at run time the
+// stores of one chunk cost 4-24 % at 256 to 32 samples.)
+template <typename T, bool SPLIT>
 __global__ __launch_bounds__(256) void gram_mfma_kernel(const cplx<T>* O, const double* w, int64_t total, int P,
-                                                        int64_t pairs, int64_t chunk, cplx<double>* part,
-                                                        cplx<double>* S) {
+                                                        int64_t pairs, int64_t chunk, cplx<double>* out) {
     extern __shared__ double lds[];   // [2][kCStage]
     const int64_t t = xcd_tile(blockIdx.x, pairs);
     if (t >= pairs) return;
-    const int64_t first = int64_t(blockIdx.y) * chunk, count = first + chunk < total ? first + chunk : total;
+    const int64_t first = SPLIT ? int64_t(blockIdx.y) * chunk : 0;
+    const int64_t count = SPLIT && first + chunk < total ? first + chunk : total;
     int ti, tj;
     upper_pair(t, ti, tj);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -188,15 +189,13 @@ __global__ __launch_bounds__(256) void gram_mfma_kernel(const cplx<T>* O, const 
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int lr = ctile_row(lane, wr, tt, r), lc2 = ctile_col(lane, wc, u);
-                if (part) {
-                    part[((int64_t(blockIdx.y) * pairs + t) * kCT + lr) * kCT + lc2] = {acc.re[tt][u][r],
-                                                                                        acc.im[tt][u][r]};
-                    continue;
-                }
                 const int gr = row0 + lr, gc = col0 + lc2;
-                if (gr < P && gc < P) {
-                    S[int64_t(gr) * P + gc] = {acc.re[tt][u][r], acc.im[tt][u][r]};
-                    if (ti != tj) S[int64_t(gc) * P + gr] = {acc.re[tt][u][r], -acc.im[tt][u][r]};
+                if constexpr (SPLIT) {
+                    out[((int64_t(blockIdx.y) * pairs + t) * kCT + lr) * kCT + lc2] = {acc.re[tt][u][r],
+                                                                                       acc.im[tt][u][r]};
+                } else if (gr < P && gc < P) {
+                    out[int64_t(gr) * P + gc] = {acc.re[tt][u][r], acc.im[tt][u][r]};
+                    if (ti != tj) out[int64_t(gc) * P + gr] = {acc.re[tt][u][r], -acc.im[tt][u][r]};
                 }
             }
 }
@@ -608,17 +607,21 @@ void launch_gram(const cplx<T>* O, const double* w, int64_t count, int P, cplx<d
     const int64_t nt = (P + kCT - 1) / kCT;
     const int64_t pairs = nt * (nt + 1) / 2;
     const size_t lds_bytes = sizeof(double) * 2 * kCStage;   // 64 KiB
-    ANN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(gram_mfma_kernel<T>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(lds_bytes)));
     const int64_t grid = (pairs + 7) / 8 * 8;
     int64_t chunk = 0;
     const int chunks = gram_chunks(P, count, &chunk);
-    gram_mfma_kernel<T><<<dim3(unsigned(grid), unsigned(chunks)), 256, lds_bytes, stream>>>(
-        O, w, count, P, pairs, chunk, chunks > 1 ? work : nullptr, S);
-    ANN_LAUNCH_CHECK();
+    auto run = [&](auto kernel, cplx<double>* out) {
+        ANN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(lds_bytes)));
+        kernel<<<dim3(unsigned(grid), unsigned(chunks)), 256, lds_bytes, stream>>>(O, w, count, P, pairs, chunk, out);
+        ANN_LAUNCH_CHECK();
+    };
     if (chunks > 1) {
+        run(gram_mfma_kernel<T, true>, work);
         gram_finish_kernel<<<unsigned(pairs * (kCT * kCT / 256)), 256, 0, stream>>>(work, chunks, P, pairs, S);
         ANN_LAUNCH_CHECK();
+    } else {
+        run(gram_mfma_kernel<T, false>, S);
     }
 }
 template void launch_gram<float>(const cplx<float>*, const double*, int64_t, int, cplx<double>*, cplx<double>*,

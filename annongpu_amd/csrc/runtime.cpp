@@ -1372,13 +1372,14 @@ void tdvp_eval_t(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with_S) {
     // S from pairs of sites and pairs of units, where they are the faster way.  With r = (N+1)^2
     // (M+1)^2 / P^2 (1 when every (site, unit), the biases' constants included, carries a parameter)
     // a sample costs them 0.019 r P^2 us / 10^6 against 0.071 for the Gram of the materialised O, but
-    // their table is gathered into S, 0.355 ((N+1)(M+1))^0.4 P^2 us / 10^6, less the 60 us that the
+    // their table is gathered into S, 0.39 ((N+1)(M+1))^0.4 P^2 us / 10^6, less the 60 us that the
     // small kernels of the other way take.  Evaluations in us, pairs and Gram: P = 16,704, 64 samples
-    // 7,007 and 2,260, 384 samples 7,938 and 8,561; P = 4,256, 64 samples 523 and 437, 192 samples
-    // 583 and 622; P = 2,144, 64 samples 238 and 293.  64 sites, 128 units, 4,096 samples: r = 1 6,852 and
-    // 21,993, r = 2.75 6,061 and 9,061, r = 3.8 5,922 and 6,611 (512 samples 1,219 and 1,073).
+    // 7,007 and 2,037, 256 samples 7,993 and 5,784, 384 samples 7,938 and 8,310; P = 4,256, 64 samples 523
+    // and 413, 256 samples 615 and 673; P = 2,144, 64 samples 238 and 286.  64 sites, 128 units,
+    // 4,096 samples: r = 1 6,852 and 21,993, r = 2.75 6,061 and 9,061, r = 3.8 5,922 and 6,611 (512
+    // samples 1,219 and 1,073).
     const double pairs = double(psi.N + 1) * (psi.M + 1), P2 = double(P) * P, r = pairs * pairs / P2;
-    bool from_pairs = with_S && r <= 3.0 && double(n) * (0.071 - 0.019 * r) >= 0.355 * std::pow(pairs, 0.4) - 60e6 / P2;
+    bool from_pairs = with_S && r <= 3.0 && double(n) * (0.071 - 0.019 * r) >= 0.39 * std::pow(pairs, 0.4) - 60e6 / P2;
     // The pairs give <O^* O'> - <O^*><O'> of uncentred sums, an error of eps (1 + |<O>|^2 / variance)
     // where the Gram of the centred O has eps; so they serve only while no parameter's mean
     // dominates.  fp64: mean squares up to the variances (a bit; 8 sites, 10 units, 2,048 samples in
