@@ -11,10 +11,11 @@
 // A flip of a 3 x 3 net reaches 25 sites: a half wave takes a chain, 2 chains a wave.
 // (The kernels of cnn.hip, which stay for other nets, hold 40 KB of activations per chain, one
 // chain per SIMD, and read a weight and an activation from LDS for every product.)
-// 12 x 12, 2 x 8 channels, fp32, against them: a sweep of 16,384 chains 64.0 -> 5.9 ms (bound by
-// the vector units: 3,456 of its instructions a pair of proposals are the products), and of 4,096
-// samples the transverse field's local energies 16.0 -> 1.85 ms, O_k 6.9 -> 0.38 ms, log psi
-// 0.72 -> 0.10 ms.
+// 12 x 12, 2 x 8 channels, fp32, against them: a sweep of 16,384 chains 64.0 -> 5.9 ms, and of 4,096
+// samples the transverse field's local energies 16.0 -> 1.85 ms, O_k 6.9 -> 0.37 ms, log psi
+// 0.72 -> 0.09 ms.  The sweep is bound by the vector units: 3,893 of their instructions a pair of
+// proposals, 3,456 of them the products, one in 3.1 cycles on every SIMD (a loop of plain multiply-adds
+// reaches one in 4.1 to 4.3); LDS bank conflicts take 11 % of the cycles.
 //
 // Every sum that a Metropolis decision depends on is taken in the order of cnn.hip's kernels:
 // input channels, then kernel sites, then output channels, then sites in increasing order over

@@ -4,9 +4,11 @@
 //
 // v_mfma_f64_16x16x4_f64 adds its four products one after the other, each with one
 // rounding (k = 0..3), so a chain of these instructions gives the sums of a scalar loop
-// over k bit for bit.  Every sum here keeps the order of such a loop: a conjugate-gradient
-// solve of 40 iterations amplifies a difference in the last bit of one product by five
-// orders of magnitude.  Lanes: A lane l = row l%16, k = l/16; B lane l = k = l/16, column
+// over k bit for bit.  theta, S V and the spin sums within a chunk of samples keep the order of such
+// a loop; the chunks are added in order, and <O>.v and O.v over threads, lanes and units in one fixed
+// order of their own.  Every one of these orders is part of the results: a conjugate-gradient solve
+// of 40 iterations amplifies a difference in the last bit of one product by five orders of
+// magnitude.  Lanes: A lane l = row l%16, k = l/16; B lane l = k = l/16, column
 // l%16; D item r of lane l = row l/16 + 4r, column l%16.
 #include "ops.hpp"
 #include "wave_net.hpp"

@@ -360,10 +360,9 @@ def cnn_quench_leg(A, steps=2, warmup=1, progress=False, precision="fp32", shift
     kms = {k: A.profiler_query(k) for k in ("mc_sweep", "local_energy", "o_k", "spin_sums", "gram", "cholesky",
                                             "log_psi")}
     sweep_ms, sweep_n = kms["mc_sweep"]
-    # work model of one single-flip proposal with local updates (a flip away from the
-    # lattice edge changes 9 layer-0 and 25 layer-1 sites): complex MACs 9*8*9 + 25*8*8*9,
-    # 8 real flops each
-    work = B * N * 8.0 * (9 * 8 * 9 + 25 * 8 * 8 * 9) * max(sweep_n, 1)
+    # work model of one single-flip proposal with local updates: the 25 second-layer sites that a
+    # flip reaches, 25*8*8*9 complex MACs of 8 real flops (the first layer is a table)
+    work = B * N * 8.0 * (25 * 8 * 8 * 9) * max(sweep_n, 1)
     E = np.array(rk.energies).real
     # the energy at the first evaluation of every step (4 evaluations per RK4 step): a
     # real-time evolution conserves it up to the Monte Carlo noise and the shift
