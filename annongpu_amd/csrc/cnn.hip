@@ -1195,9 +1195,11 @@ void launch_generic_mc(const V& net, uint64_t* chain_confs, int words, int num_c
     using T = typename V::real_t;
     if constexpr (std::is_same<V, CnnView<T>>::value) {
         // (a net is refused by its size alone, whatever kernels serve it)
-        check_lds(cnn_inc_lds(net) + cnn_stage_bytes(net));
-        if (cnn_pair_mc(net, chain_confs, words, num_chains, move, num_proposals, counter, seed, accepted, stream)) return;
         const int stage = cnn_stage_bytes(net);
+        check_lds(cnn_inc_lds(net) + stage);
+        if (cnn_pair_mc(net, chain_confs, words, num_chains, move, num_proposals, counter, seed, accepted,
+                        cnn_inc_lds(net) + stage, stream))
+            return;
         dispatch_vmax(net, [&](auto vt) {
             constexpr int VM = decltype(vt)::value;
             auto run = [&](auto kern) {
@@ -1226,9 +1228,9 @@ void launch_generic_local_energy(const V& net, const OpView& op, const uint64_t*
     if (count <= 0) return;
     using T = typename V::real_t;
     if constexpr (std::is_same<V, CnnView<T>>::value) {
-        check_lds(cnn_inc_lds(net) + cnn_stage_bytes(net));
-        if (cnn_pair_local_energy(net, op, confs, count, e_loc, stream)) return;
         const int stage = cnn_stage_bytes(net);
+        check_lds(cnn_inc_lds(net) + stage);
+        if (cnn_pair_local_energy(net, op, confs, count, e_loc, cnn_inc_lds(net) + stage, stream)) return;
         dispatch_vmax(net, [&](auto vt) {
             constexpr int VM = decltype(vt)::value;
             auto run = [&](auto kern) {

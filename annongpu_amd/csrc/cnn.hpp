@@ -120,16 +120,17 @@ struct ClassicalView {
 };
 
 // The kernels of cnn_pair.hip; false (and nothing launched) where they do not serve the net, the
-// move or the operator
+// move or the operator, or where the general kernel, which takes general_lds bytes of LDS a chain or
+// sample, is the faster one
 template <typename T>
 bool cnn_pair_log_psi(const CnnView<T>& v, const uint64_t* confs, int words, int64_t count, cplx<double> lp,
                       cplx<double>* log_psi, double* weight, hipStream_t stream);
 template <typename T>
 bool cnn_pair_mc(const CnnView<T>& v, uint64_t* chain_confs, int words, int num_chains, int move, int64_t num_proposals,
-                 uint64_t counter, uint64_t seed, uint32_t* accepted, hipStream_t stream);
+                 uint64_t counter, uint64_t seed, uint32_t* accepted, size_t general_lds, hipStream_t stream);
 template <typename T>
 bool cnn_pair_local_energy(const CnnView<T>& v, const OpView& op, const uint64_t* confs, int64_t count,
-                           cplx<double>* e_loc, hipStream_t stream);
+                           cplx<double>* e_loc, size_t general_lds, hipStream_t stream);
 template <typename T>
 bool cnn_pair_ok(const CnnView<T>& v, const uint64_t* confs, int words, int64_t count, cplx<T>* O, hipStream_t stream);
 

@@ -662,6 +662,17 @@ size_t pair_energy_lds(const CnnPair<T>& f, int tpw, int G) {
            sizeof(uint16_t) * G;
 }
 
+// Rounds of 64 lanes in which the general kernels take the outputs that `reached` changed sites
+// have: their lanes hold (site, channel) pairs, the lanes here sites with the channels one after
+// another.  So for many channels at few sites and no more chains (samples) than the general kernels
+// hold at once, `resident`, those are the faster ones (beyond, the more chains in flight here win: 32
+// sites, kernels of 3, 4,096 chains, 24 channels 2.2 times, 12 channels 1.5 times).
+template <typename T>
+int general_rounds(const CnnPair<T>& f, int reached) {
+    return (reached * f.C1 + 63) / 64;
+}
+int64_t resident(size_t general_lds) { return 256 * std::max<int64_t>(1, 160 * 1024 / int64_t(general_lds)); }
+
 }  // namespace
 
 template <typename T>
@@ -684,9 +695,15 @@ bool cnn_pair_log_psi(const CnnView<T>& v, const uint64_t* confs, int words, int
 
 template <typename T>
 bool cnn_pair_mc(const CnnView<T>& v, uint64_t* chain_confs, int words, int num_chains, int move, int64_t num_proposals,
-                 uint64_t counter, uint64_t seed, uint32_t* accepted, hipStream_t stream) {
+                 uint64_t counter, uint64_t seed, uint32_t* accepted, size_t general_lds, hipStream_t stream) {
     const CnnPair<T>& f = v.pair;
     if (!f.wf || (move != MOVE_FLIP && move != MOVE_EXCHANGE)) return false;
+    // Two rounds for a block of 8 channels is where both take as long: 100 chains in fp32, flips of 32
+    // sites, here against there, kernels of 3 (5 sites reached), 8 channels 176 and 247 us, 12 channels
+    // 475 and 308, 32 channels 2,817 and 1,634; kernels of 3 x 3 (25 reached), 12 channels 2,580 and 2,580,
+    // 16 channels 3,403 and 6,091.
+    const int reached = (move == MOVE_EXCHANGE ? 2 : 1) * f.n1;
+    if (f.C1 > 8 && num_chains <= resident(general_lds) && general_rounds(f, reached) < 2 * f.blocks) return false;
     const bool half = move == MOVE_FLIP && f.n1 <= 32;
     // a lane per reached site of one or two flips
     if ((move == MOVE_EXCHANGE ? 2 : 1) * f.n1 > 64 || f.n0 > (half ? 32 : 64)) return false;
@@ -713,9 +730,16 @@ bool cnn_pair_mc(const CnnView<T>& v, uint64_t* chain_confs, int words, int num_
 
 template <typename T>
 bool cnn_pair_local_energy(const CnnView<T>& v, const OpView& op, const uint64_t* confs, int64_t count,
-                           cplx<double>* e_loc, hipStream_t stream) {
+                           cplx<double>* e_loc, size_t general_lds, hipStream_t stream) {
     const CnnPair<T>& f = v.pair;
     if (!f.wf || op.max_flips > 2 || op.num_groups > kPList) return false;
+    // as for the chains; two flips at a time are on a par at three rounds a block of channels (512
+    // samples, 31 bonds, kernels of 5: 12 channels 443 and 350 us, of 3 x 3: 1.35 times), pairs of single
+    // flips at half a round (32 channels, kernels of 2 in fp64: 1,190 and 1,024 us)
+    const int rounds = general_rounds(f, std::max(op.max_flips, 1) * f.n1);
+    if (f.C1 > 8 && count <= resident(general_lds) &&
+        (op.max_flips == 2 ? rounds < 3 * f.blocks : f.blocks >= 4 && 2 * rounds <= f.blocks))
+        return false;
     const bool half = op.max_flips <= 1 && f.n1 <= 32;
     if ((op.max_flips == 2 ? 2 : 1) * f.n1 > 64 || f.n0 > (half ? 32 : 64)) return false;
     const size_t lds = pair_energy_lds(f, half ? 2 : 1, op.num_groups);
@@ -740,6 +764,11 @@ template <typename T>
 bool cnn_pair_ok(const CnnView<T>& v, const uint64_t* confs, int words, int64_t count, cplx<T>* O, hipStream_t stream) {
     const CnnPair<T>& f = v.pair;
     if (!f.wf || f.C0 * f.v0 > kOThreads) return false;
+    // A workgroup per sample waits 5 us at its barriers whatever the net; a net of few products is the
+    // faster on the general kernel's single waves where there are many samples: 40 sites, 5,000 samples, one
+    // channel, kernels of 2, here against there 69 and 14 us, 3 channels, kernels of 5, 86 and 84, 4
+    // channels 103 and 134; 600 samples, one channel 18 and 10, 4 channels 24 and 88.
+    if (125 * int64_t(f.C0) * f.C1 * f.v1 * std::max(f.N, 64) < 64 * std::min<int64_t>(5000, count)) return false;
     const size_t lds = pair_ok_lds(f);
     if (lds > kPLds) return false;
     dispatch_pair(f, [&](auto cb, auto vm) {
@@ -757,9 +786,9 @@ bool cnn_pair_ok(const CnnView<T>& v, const uint64_t* confs, int words, int64_t 
     template bool cnn_pair_log_psi<T>(const CnnView<T>&, const uint64_t*, int, int64_t, cplx<double>, cplx<double>*,  \
                                       double*, hipStream_t);                                                           \
     template bool cnn_pair_mc<T>(const CnnView<T>&, uint64_t*, int, int, int, int64_t, uint64_t, uint64_t, uint32_t*, \
-                                 hipStream_t);                                                                         \
+                                 size_t, hipStream_t);                                                                 \
     template bool cnn_pair_local_energy<T>(const CnnView<T>&, const OpView&, const uint64_t*, int64_t, cplx<double>*, \
-                                           hipStream_t);                                                               \
+                                           size_t, hipStream_t);                                                       \
     template bool cnn_pair_ok<T>(const CnnView<T>&, const uint64_t*, int, int64_t, cplx<T>*, hipStream_t);
 ANN_CNN_PAIR_INSTANTIATE(float)
 ANN_CNN_PAIR_INSTANTIATE(double)

@@ -8,7 +8,8 @@ Shapes: kernels of 1 to 9 sites in one to three dimensions, kernels as wide as t
 read twice), 256 sites, odd channel numbers and channel blocks of 2, 4 and 8, flips that reach more
 and fewer than 32 sites, exchange moves, operators of one and two flips.  The last shape's flips reach
 45 sites: one flip is served, two are not (more than 64).  A lattice of one site has one class only and
-is compared with the oracle.
+is compared with the oracle.  Which kernels take a call may depend on the number of chains or samples;
+both give a chain the same configurations and a sample the same values.
 
 Tolerances: a pre-activation is a sum of K <= C0 v1 products of size below 1, log psi one of N C1
 outputs, O_k one of N products: 8 eps per sum's square root of terms, relative to the largest value
@@ -160,3 +161,40 @@ def test_one_site(precision):
     if precision == "fp64":
         run = orc.mc_run(o, 5, 3, 2, 3, move=orc.MOVE_FLIP, seed=8)
         assert np.array_equal(mc.last_samples()[:, 0], run["samples"][:, 0])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_few_and_many(precision):
+    """sixteen channels at five sites: few chains and samples take the general kernels, many these; one
+    channel: many samples' O_k take the general kernel"""
+    import annongpu_amd as A
+    N, [psi, _] = nets([1, 1, 20], [(16, [1, 1, 3]), (16, [1, 1, 3])], precision, 3)
+    eps = np.finfo(np.float64 if precision == "fp64" else np.float32).eps
+    few, many = 8, 5000
+
+    def chains(p, n, move):
+        ens = A.MonteCarloSpins(n, 1, 2, n, move=move, seed=5)
+        A.log_psi(p, ens)
+        return ens.last_samples()[:few]
+
+    for move in ("flip", "exchange"):
+        [a] = served("mc", [psi], lambda p: chains(p, few, move), 0)
+        [b] = served("mc", [psi], lambda p: chains(p, many, move))
+        assert np.array_equal(a, b)
+    rng = np.random.default_rng(1)
+    confs = words(N, many, rng)
+    op = operators(A, N)[1]
+    [a] = served("local_energy", [psi], lambda p: A.local_energies(op, p, A.SampleList(N, confs[:few])), 0)
+    [b] = served("local_energy", [psi], lambda p: A.local_energies(op, p, A.SampleList(N, confs)))
+    terms = N * 16 + 16 * 3
+    assert np.abs(a - b[:few]).max() <= 8 * eps * terms * np.abs(a).max()
+    N, [psi, _] = nets([1, 1, 20], [(1, [1, 1, 3]), (1, [1, 1, 3])], precision, 4)
+
+    def samples(p, n):
+        t = A.TDVP(p.num_params)
+        t.eval_F(operators(A, N)[0], p, A.SampleList(N, confs[:n]))
+        return t.O_k_samples[:few]
+
+    [a] = served("ok", [psi], lambda p: samples(p, few))
+    [b] = served("ok", [psi], lambda p: samples(p, many), 0)
+    assert np.abs(a - b).max() <= 8 * eps * np.sqrt(N + 3) * np.abs(a).max()
