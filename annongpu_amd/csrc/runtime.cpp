@@ -1382,11 +1382,12 @@ void tdvp_eval_t(Tdvp& t, Operator& op, Psi& psi, Ensemble& ens, bool with_S) {
     bool from_pairs = with_S && r <= 3.0 && double(n) * (0.071 - 0.019 * r) >= 0.39 * std::pow(pairs, 0.4) - 60e6 / P2;
     // The pairs give <O^* O'> - <O^*><O'> of uncentred sums, an error of eps (1 + |<O>|^2 / variance)
     // where the Gram of the centred O has eps; so they serve only while no parameter's mean
-    // dominates.  fp64: mean squares up to the variances (a bit; 8 sites, 10 units, 2,048 samples in
-    // one chain against long double: 8e-15 and 9e-15 of the variance at a ratio of 0.9, 3.9e-14 and
-    // 7.8e-13 at 14).  fp32: up to 2e-13 of the variance, far below the fp32 rounding of O.
+    // dominates.  fp64: mean squares up to twice the variances (a bit; 8 sites, 10 units, 2,048 samples
+    // in one chain against long double, centred and pairs: 6e-15 and 9e-15 of the variance at a ratio of
+    // 0.7, 1.3e-14 and 2.1e-14 at 1.6, 3.9e-14 and 7.8e-13 at 14).  fp32: up to 2e-13 of the variance, far
+    // below the fp32 rounding of O.
     if (from_pairs)
-        launch_mean_dominated(t.Obar.p, t.diag.p, P, sizeof(T) == 8 ? 1.0 : 1024.0, t.sums.p + 4, S());
+        launch_mean_dominated(t.Obar.p, t.diag.p, P, sizeof(T) == 8 ? 2.0 : 1024.0, t.sums.p + 4, S());
     // E, E2 and sum w go to page-locked memory; the host reads them, and <O> and F,
     // when they are asked for (the evaluation returns without synchronising, so a
     // solve that follows is queued behind it at once)

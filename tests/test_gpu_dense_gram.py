@@ -5,7 +5,7 @@ words) and over the layouts that reach it, sample counts and weights that do not
 The O_k samples are exact copies of what S is built from, so both sides are fp64 sums of the
 same products: |S - S_ref| <= 4 n eps max|sum w |O_k|^2| entrywise (n summands).
 
-The pairs serve while no parameter's squared mean exceeds its variance (fp32: 1,024 times it); where
+The pairs serve while no parameter's squared mean exceeds twice its variance (fp32: 1,024 times it); where
 one does, S comes from the centred O_k and its error stays within the rounding of the n products and
 of the centring, relative to the two parameters' spreads."""
 import ctypes
@@ -68,7 +68,7 @@ def test_dense_gram(kind, N, M, n, precision):
     t, pairs = evaluate(A, psi, A.Operator(1.0 * A.sigma_z(0)), A.SampleList(N, confs, w))
     O = t.O_k_samples
     if n > 1:
-        assert pairs == (dominance(O, w) <= (1 if precision == "fp64" else 1024))
+        assert pairs == (dominance(O, w) <= (2 if precision == "fp64" else 1024))
     mean = w @ O
     S = (O.conj() * w[:, None]).T @ O - np.outer(mean.conj(), mean)
     assert np.abs(t.S_matrix - S).max() <= 4 * max(n, 8) * np.finfo(float).eps * (w @ np.abs(O) ** 2).max()
@@ -94,7 +94,7 @@ def test_dominating_means(bias, flips, precision):
     O = t.O_k_samples.astype(np.clongdouble)
     w = np.full(n, 1 / n)
     ratio = dominance(O.astype(complex), w)
-    assert pairs == (ratio <= (1 if precision == "fp64" else 1024))
+    assert pairs == (ratio <= (2 if precision == "fp64" else 1024))
     x = O - O.mean(0)
     S = (x.conj().T @ x) / n
     spread = np.sqrt(np.diag(S).real)
