@@ -21,7 +21,7 @@
 // -2 (W_b + W_a), where an operator needs them); d is +-D.  Per unit a lane reads the sample's 24
 // bytes once and 8 bytes for each of its two terms.  The unit sums are taken per tile in fp32 and
 // over the tiles in fp64.
-// Bound by the vector units: 0.76 of their issue slots, LDS bank conflicts in 16 % of the cycles.
+// Bound by the vector units: 0.83 of their issue slots, LDS bank conflicts in 16 % of the cycles.
 // 10x10 Heisenberg, 400 units, 16,384 samples, fp32: 1,205 -> 565 us.  With few terms for the units
 // the general kernel is the faster one: local_energy_terms_serves.
 #include "kernels.hpp"
